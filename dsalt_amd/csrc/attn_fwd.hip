@@ -672,12 +672,36 @@ __global__ __launch_bounds__(64 * NW, ((sizeof(T) == 2 && D == 64 && RG == 2 && 
 // stay within one landmark set, block_size a multiple of 128); for 16-bit head_dim 128, two
 // row groups per wave (FWD_RG2, same condition) or 64-key chunks instead of 32 (FWD_BN64;
 // ignored with FWD_RG2);
-// fp32 takes its single compiled tiling.  Sets of more than kSetSlots landmarks, and
+// fp32 takes its single compiled tiling.  With no forward bit set the operator picks by the work
+// in 64-row tiles, tokens x heads / 64 (one call, plan included, against the 64-row tiling of
+// 64-key, at head_dim 128 32-key, chunks; windows up to 64 .. 512, 16 .. 256 landmarks):
+//   head_dim 64: FWD_RG2 | FWD_BN32 from kRg2Tiles on.  The 128-row blocks read each K and V^T
+//     operand from LDS once for 32 rows (the 64-row tiling reads 1 KB of LDS per MFMA), but below
+//     that there are too few of them: 1024 tiles 1.04-1.07x the time, 1536 0.90-0.96x, 2048
+//     0.86-0.95x, 8192 0.80-0.82x (16 heads x 32768, windows up to 512: 153.5 -> 123.1 us);
+//   head_dim 128: FWD_8W from kW8Tiles on, where staging the key chunks bounds the kernel: 32768
+//     tiles 0.945-0.997x (16 heads x 131072, 256 landmarks: 1130 -> 1077 us); 8192 tiles
+//     0.93-1.12x and 2048 0.96-1.07x (slower for windows below 512), so these keep four waves.
+// The training variant keeps its 64-row tiling (with RG2 its edge terms spill: 189 -> 335 us).
+// Sets of more than kSetSlots landmarks, and
 // block-causal sets of a block_size that is not a multiple of 64, take the default tiling's
 // wide instantiation (variant bits ignored).
+constexpr int64_t kRg2Tiles = 1536, kW8Tiles = 16384;
+
+// the forward tiling bits the call runs with: its own, or the rule's when it names none
+template <typename T, int D, bool TR>
+static int fwd_variant(const AttnParams& p) {
+    constexpr int kFwdBits = DSALT_VARIANT_FWD_BN32 | DSALT_VARIANT_FWD_RG2 | DSALT_VARIANT_FWD_BN64 | DSALT_VARIANT_FWD_8W;
+    if (TR || sizeof(T) != 2 || (p.variant & kFwdBits) || p.block_size % 128) return p.variant;
+    const int64_t tiles = (int64_t)p.total_len * p.n_heads / 64;
+    if (D == 64) return tiles >= kRg2Tiles ? p.variant | DSALT_VARIANT_FWD_RG2 | DSALT_VARIANT_FWD_BN32 : p.variant;
+    return tiles >= kW8Tiles ? p.variant | DSALT_VARIANT_FWD_8W : p.variant;
+}
+
 template <typename T, int D, bool TR>
 static void fwd_run(const AttnParams& p, hipStream_t stream) {
     constexpr int BN = FwdShape<T, D>::BN;
+    const int variant = fwd_variant<T, D, TR>(p);
     if constexpr (!TR) {
         if (p.block_size % 64 || p.k_lmk > kSetSlots) {
             DSALT_LAUNCH("attn_fwd", (fwd_kernel<T, D, BN, 1, false, true>), dim3(p.n_heads * p.num_seqs * p.n_tiles),
@@ -686,10 +710,10 @@ static void fwd_run(const AttnParams& p, hipStream_t stream) {
         }
     }
     if constexpr (sizeof(T) == 2) {
-        const bool rg2 = (p.variant & DSALT_VARIANT_FWD_RG2) != 0 && (p.block_size == 0 || p.block_size % 128 == 0);
+        const bool rg2 = (variant & DSALT_VARIANT_FWD_RG2) != 0 && (p.block_size == 0 || p.block_size % 128 == 0);
         const int total = p.n_heads * p.num_seqs * ceil_div(p.n_tiles, rg2 ? 2 : 1);
         if constexpr (D == 64) {
-            const bool bn32 = (p.variant & DSALT_VARIANT_FWD_BN32) != 0;
+            const bool bn32 = (variant & DSALT_VARIANT_FWD_BN32) != 0;
             if (rg2) {
                 if (bn32) DSALT_LAUNCH("attn_fwd", (fwd_kernel<T, D, 32, 2, TR>), dim3(total), dim3(256), 0, stream, p);
                 else DSALT_LAUNCH("attn_fwd", (fwd_kernel<T, D, BN, 2, TR>), dim3(total), dim3(256), 0, stream, p);
@@ -701,8 +725,8 @@ static void fwd_run(const AttnParams& p, hipStream_t stream) {
             }
         } else if constexpr (!TR) {  // head_dim 128 (inference shapes)
             // two row groups keep 32-key chunks (with 64-key chunks they would spill at 256 VGPRs)
-            const bool bn64 = (p.variant & DSALT_VARIANT_FWD_BN64) != 0;
-            const bool w8 = (p.variant & DSALT_VARIANT_FWD_8W) != 0 && (p.block_size == 0 || p.block_size % 128 == 0);
+            const bool bn64 = (variant & DSALT_VARIANT_FWD_BN64) != 0;
+            const bool w8 = (variant & DSALT_VARIANT_FWD_8W) != 0 && (p.block_size == 0 || p.block_size % 128 == 0);
             if (w8) {
                 DSALT_LAUNCH("attn_fwd", (fwd_kernel<T, D, BN, 1, TR, false, 8>),
                              dim3(p.n_heads * p.num_seqs * ceil_div(p.n_tiles, 2)), dim3(512), 0, stream, p);
@@ -723,13 +747,16 @@ static void fwd_run(const AttnParams& p, hipStream_t stream) {
 }
 
 template <typename T>
-static hipError_t fwd_dispatch(const AttnParams& p, bool plan_ready, hipStream_t stream) {
+static hipError_t fwd_dispatch(AttnParams p, bool plan_ready, hipStream_t stream) {
     if (p.n_heads * p.num_seqs * p.n_tiles == 0) return hipSuccess;
     if (!plan_ready) {
         const hipError_t e = plan_launch(p, stream);
         if (e != hipSuccess) return e;
     }
-    const bool tr = p.w_cont != nullptr;
+    // without a soft edge every band key's bias is 0: the training forward is the operator over
+    // the integer windows, in the operator's tiling
+    const bool tr = p.w_cont != nullptr && p.edge > 0.f;
+    if (!tr) p.w_cont = nullptr;
     if (p.head_dim == 64) {
         if (tr) fwd_run<T, 64, true>(p, stream);
         else fwd_run<T, 64, false>(p, stream);
