@@ -111,6 +111,11 @@ class SiluMulArgs(ctypes.Structure):
                 ("up", _vp), ("up_stride", _i64), ("out", _vp), ("out_stride", _i64)]
 
 
+class SortArgs(ctypes.Structure):
+    _fields_ = [("n_sets", _i64), ("k", _i32), ("idx_bytes", _i32), ("idx", _vp), ("sorted", _vp), ("perm", _vp),
+                ("bias", _vp), ("bias_sorted", _vp), ("bias_bytes", _i32)]
+
+
 class GatherArgs(ctypes.Structure):
     _fields_ = [("p", Problem),
                 ("k", _vp), ("k_stride_t", _i64), ("k_stride_h", _i64),
@@ -130,6 +135,10 @@ SIGNATURES = {
     "dsalt_fwd_workspace_bytes": ([ctypes.POINTER(FwdArgs)], _sz),
     "dsalt_fwd": ([ctypes.POINTER(FwdArgs), _vp], ctypes.c_int),
     "dsalt_fwd_noalloc": ([ctypes.POINTER(FwdArgs), _vp], ctypes.c_int),
+    "dsalt_fwd_f32out": ([ctypes.POINTER(FwdArgs), _vp, _vp], ctypes.c_int),
+    "dsalt_bwd_f32dout": ([ctypes.POINTER(BwdArgs), _vp, _i64, _i64, _vp], ctypes.c_int),
+    "dsalt_train_fwd_f32out": ([ctypes.POINTER(TrainFwdArgs), _vp, _vp], ctypes.c_int),
+    "dsalt_train_bwd_f32dout": ([ctypes.POINTER(TrainBwdArgs), _vp, _i64, _i64, _vp], ctypes.c_int),
     "dsalt_bwd_workspace_bytes": ([ctypes.POINTER(BwdArgs)], _sz),
     "dsalt_bwd": ([ctypes.POINTER(BwdArgs), _vp], ctypes.c_int),
     "dsalt_gather_landmarks": ([ctypes.POINTER(GatherArgs), _vp], ctypes.c_int),
@@ -139,6 +148,7 @@ SIGNATURES = {
     "dsalt_train_bwd": ([ctypes.POINTER(TrainBwdArgs), _vp], ctypes.c_int),
     "dsalt_rope_qk": ([ctypes.POINTER(RopeArgs), _vp], ctypes.c_int),
     "dsalt_silu_mul": ([ctypes.POINTER(SiluMulArgs), _vp], ctypes.c_int),
+    "dsalt_sort_landmarks": ([ctypes.POINTER(SortArgs), _vp], ctypes.c_int),
     "dsalt_export_probs": ([ctypes.POINTER(ProbsArgs), _vp], ctypes.c_int),
     "dsalt_cross_entropy_rows": ([ctypes.POINTER(CeArgs), _vp], ctypes.c_int),
     "dsalt_timing_enable": ([ctypes.c_int], ctypes.c_int),

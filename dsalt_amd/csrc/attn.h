@@ -29,6 +29,9 @@ struct AttnParams {
     int64_t o_st, o_sh;
     const void* dout;
     int64_t do_st, do_sh;
+    float* out32;            // forward: the output's rounded values as float32 too, [T, H, D], or null
+    const float* do32;       // backward: the upstream gradient in float32 (strides do32_st, do32_sh), or
+    int64_t do32_st, do32_sh;  // null; the dQ pass rounds it into `dout`, which the later passes read
     const float* lse;        // [T, H]
     float* lse_out;
     const int32_t* w;

@@ -154,7 +154,17 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 && D == 64) ? (BN == 32 ? (TR 
     const T* ohead = (const T*)p.o + (int64_t)st * p.o_st + (int64_t)h * p.o_sh;
     RowReg<T, D> qr, dor, orr;
     qr.load(valid ? qhead + (int64_t)i * p.q_st : nullptr, qhead, g);
-    dor.load(valid ? dohead + (int64_t)i * p.do_st : nullptr, dohead, g);
+    if constexpr (kHalf) {
+        if (p.do32) {
+            const float* d0 = p.do32 + (int64_t)st * p.do32_st + (int64_t)h * p.do32_sh;
+            load_rounded<T, D>(dor.x, valid ? d0 + (int64_t)i * p.do32_st : nullptr, d0,
+                               const_cast<T*>(dohead) + (int64_t)i * p.do_st, g);
+        } else {
+            dor.load(valid ? dohead + (int64_t)i * p.do_st : nullptr, dohead, g);
+        }
+    } else {
+        dor.load(valid ? dohead + (int64_t)i * p.do_st : nullptr, dohead, g);
+    }
     orr.load(valid ? ohead + (int64_t)i * p.o_st : nullptr, ohead, g);
     // the band's key range, clamped to the sequence: a plan made for other windows or offsets
     // gives wrong values, never reads outside the sequence's rows

@@ -662,6 +662,9 @@ __global__ __launch_bounds__(64 * NW, ((sizeof(T) == 2 && D == 64 && RG == 2 && 
         SR::run(stage, acc[u], rg[u].valid ? 1.0f / l_tot : 0.f, lane, [&](int rr) {
             const int ir = __shfl(vi, rr);
             return ir >= 0 ? o0 + (int64_t)ir * p.o_st : (T*)nullptr;
+        }, [&](int rr) {
+            const int ir = p.out32 ? __shfl(vi, rr) : -1;
+            return ir >= 0 ? p.out32 + ((int64_t)(st + ir) * p.n_heads + h) * D : (float*)nullptr;
         });
         if (rg[u].valid && g == 0) p.lse_out[(int64_t)(st + rg[u].i) * p.n_heads + h] = m_run[u] * p.scale + __logf(l_tot);
     }

@@ -13,6 +13,7 @@
 #include "probs.h"
 #include "rope.h"
 #include "select.h"
+#include "sets.h"
 #include "common.h"
 
 namespace {
@@ -274,21 +275,36 @@ size_t dsalt_plan_bytes(const dsalt_problem* p) {
     return dsalt::plan_bytes(attn_common(*p, 1.0f));
 }
 
+static int check_f32out(const dsalt_fwd_args* a, const float* out_f32) {
+    if (!out_f32 || !aligned16(out_f32)) return fail(DSALT_ERR_INVALID, "out_f32 must be non-null and 16-byte aligned");
+    if (a->p.dtype == DSALT_DTYPE_F32) return fail(DSALT_ERR_UNSUPPORTED, "out_f32 goes with 16-bit tensors");
+    return DSALT_OK;
+}
+
 // the forward's only workspace is the row plan, which a caller-given plan buffer replaces
 size_t dsalt_fwd_workspace_bytes(const dsalt_fwd_args* a) {
     if (!a || check_problem(a->p, true)) return 0;
     return a->plan ? 0 : dsalt::plan_bytes(attn_common(a->p, 1.0f));
 }
 
-int dsalt_fwd(const dsalt_fwd_args* a, dsalt_stream_t stream) {
+static int fwd_call(const dsalt_fwd_args* a, float* out32, dsalt_stream_t stream) {
     dsalt::AttnParams p;
     int rc = fwd_params(a, true, &p);
     if (rc) return rc;
+    p.out32 = out32;
     const size_t need = a->plan ? 0 : dsalt::plan_bytes(p);
     if (need && (!a->workspace || a->workspace_bytes < need))
         return fail(DSALT_ERR_WORKSPACE, "forward needs %zu workspace bytes, got %zu", need, a->workspace_bytes);
     return hip_status(dsalt::fwd_launch(p, a->workspace, a->plan, a->plan_ready != 0, (hipStream_t)stream),
                       "dsalt_fwd");
+}
+
+int dsalt_fwd(const dsalt_fwd_args* a, dsalt_stream_t stream) { return fwd_call(a, nullptr, stream); }
+
+int dsalt_fwd_f32out(const dsalt_fwd_args* a, float* out_f32, dsalt_stream_t stream) {
+    if (!a) return fail(DSALT_ERR_INVALID, "null argument struct");
+    const int rc = check_f32out(a, out_f32);
+    return rc ? rc : fwd_call(a, out_f32, stream);
 }
 
 }  // extern "C"
@@ -362,12 +378,13 @@ size_t dsalt_train_fwd_workspace_bytes(const dsalt_train_fwd_args* a) {
     return wint_bytes(p) + (a->base.plan ? 0 : dsalt::plan_bytes(p));
 }
 
-int dsalt_train_fwd(const dsalt_train_fwd_args* a, dsalt_stream_t stream) {
+static int train_fwd_call(const dsalt_train_fwd_args* a, float* out32, dsalt_stream_t stream) {
     if (!a) return fail(DSALT_ERR_INVALID, "null argument struct");
     dsalt::AttnParams p;
     int rc = fwd_params(&a->base, false, &p);
     if (rc) return rc;
     if ((rc = train_params(a->w_cont, a->tau_win, a->win_edge, &p))) return rc;
+    p.out32 = out32;
     const size_t need = wint_bytes(p) + (a->base.plan ? 0 : dsalt::plan_bytes(p));
     if (!a->base.workspace || a->base.workspace_bytes < need)
         return fail(DSALT_ERR_WORKSPACE, "training forward needs %zu workspace bytes, got %zu", need,
@@ -378,6 +395,14 @@ int dsalt_train_fwd(const dsalt_train_fwd_args* a, dsalt_stream_t stream) {
     if (e == hipSuccess)
         e = dsalt::fwd_launch(p, (char*)a->base.workspace + wint_bytes(p), a->base.plan, false, (hipStream_t)stream);
     return hip_status(e, "dsalt_train_fwd");
+}
+
+int dsalt_train_fwd(const dsalt_train_fwd_args* a, dsalt_stream_t stream) { return train_fwd_call(a, nullptr, stream); }
+
+int dsalt_train_fwd_f32out(const dsalt_train_fwd_args* a, float* out_f32, dsalt_stream_t stream) {
+    if (!a) return fail(DSALT_ERR_INVALID, "null argument struct");
+    const int rc = check_f32out(&a->base, out_f32);
+    return rc ? rc : train_fwd_call(a, out_f32, stream);
 }
 
 static int bwd_params(const dsalt_bwd_args* a, dsalt::AttnParams* out, bool need_w = true) {
@@ -431,20 +456,41 @@ static int bwd_params(const dsalt_bwd_args* a, dsalt::AttnParams* out, bool need
     return DSALT_OK;
 }
 
+// a float32 upstream gradient: rows of 16-byte vectors; `dout` receives its rounded values
+static int check_f32dout(const dsalt_bwd_args* a, const float* d, int64_t st, int64_t sh) {
+    if (a->p.dtype == DSALT_DTYPE_F32) return fail(DSALT_ERR_UNSUPPORTED, "dout_f32 goes with 16-bit tensors");
+    if (!d || !aligned16(d) || st <= 0 || sh < 0 || st % 4 || sh % 4)
+        return fail(DSALT_ERR_INVALID, "dout_f32 needs 16-byte aligned rows with positive strides (%lld, %lld)",
+                    (long long)st, (long long)sh);
+    return DSALT_OK;
+}
+
 size_t dsalt_bwd_workspace_bytes(const dsalt_bwd_args* a) {
     dsalt::AttnParams p;
     if (bwd_params(a, &p)) return 0;
     return dsalt::bwd_workspace(p, a->plan != nullptr);
 }
 
-int dsalt_bwd(const dsalt_bwd_args* a, dsalt_stream_t stream) {
+static int bwd_call(const dsalt_bwd_args* a, const float* do32, int64_t st, int64_t sh, dsalt_stream_t stream) {
     dsalt::AttnParams p;
     int rc = bwd_params(a, &p);
     if (rc) return rc;
+    p.do32 = do32;
+    p.do32_st = st;
+    p.do32_sh = sh;
     size_t need = dsalt::bwd_workspace(p, a->plan != nullptr);
     if (!a->workspace || a->workspace_bytes < need || !aligned16(a->workspace))
         return fail(DSALT_ERR_WORKSPACE, "backward needs %zu workspace bytes, got %zu", need, a->workspace_bytes);
     return hip_status(dsalt::bwd_launch(p, a->workspace, a->plan, (hipStream_t)stream), "dsalt_bwd");
+}
+
+int dsalt_bwd(const dsalt_bwd_args* a, dsalt_stream_t stream) { return bwd_call(a, nullptr, 0, 0, stream); }
+
+int dsalt_bwd_f32dout(const dsalt_bwd_args* a, const float* dout_f32, int64_t stride_t, int64_t stride_h,
+                      dsalt_stream_t stream) {
+    if (!a) return fail(DSALT_ERR_INVALID, "null argument struct");
+    const int rc = check_f32dout(a, dout_f32, stride_t, stride_h);
+    return rc ? rc : bwd_call(a, dout_f32, stride_t, stride_h, stream);
 }
 
 // training backward workspace: integer windows, per-head d w~, then the operator's
@@ -458,12 +504,16 @@ size_t dsalt_train_bwd_workspace_bytes(const dsalt_train_bwd_args* a) {
     return train_bwd_extra(p) + dsalt::bwd_workspace(p, a->base.plan != nullptr);
 }
 
-int dsalt_train_bwd(const dsalt_train_bwd_args* a, dsalt_stream_t stream) {
+static int train_bwd_call(const dsalt_train_bwd_args* a, const float* do32, int64_t st, int64_t sh,
+                          dsalt_stream_t stream) {
     if (!a) return fail(DSALT_ERR_INVALID, "null argument struct");
     dsalt::AttnParams p;
     int rc = bwd_params(&a->base, &p, false);
     if (rc) return rc;
     if ((rc = train_params(a->w_cont, a->tau_win, a->win_edge, &p))) return rc;
+    p.do32 = do32;
+    p.do32_st = st;
+    p.do32_sh = sh;
     if (!a->d_w) return fail(DSALT_ERR_INVALID, "d_w is required");
     const size_t need = train_bwd_extra(p) + dsalt::bwd_workspace(p, a->base.plan != nullptr);
     if (!a->base.workspace || a->base.workspace_bytes < need || !aligned16(a->base.workspace))
@@ -478,6 +528,17 @@ int dsalt_train_bwd(const dsalt_train_bwd_args* a, dsalt_stream_t stream) {
     if (e == hipSuccess) e = dsalt::bwd_launch(p, w + train_bwd_extra(p), a->base.plan, (hipStream_t)stream);
     if (e == hipSuccess) e = dsalt::train_dw_launch(p, (hipStream_t)stream);
     return hip_status(e, "dsalt_train_bwd");
+}
+
+int dsalt_train_bwd(const dsalt_train_bwd_args* a, dsalt_stream_t stream) {
+    return train_bwd_call(a, nullptr, 0, 0, stream);
+}
+
+int dsalt_train_bwd_f32dout(const dsalt_train_bwd_args* a, const float* dout_f32, int64_t stride_t, int64_t stride_h,
+                            dsalt_stream_t stream) {
+    if (!a) return fail(DSALT_ERR_INVALID, "null argument struct");
+    const int rc = check_f32dout(&a->base, dout_f32, stride_t, stride_h);
+    return rc ? rc : train_bwd_call(a, dout_f32, stride_t, stride_h, stream);
 }
 
 int dsalt_rope_qk(const dsalt_rope_args* a, dsalt_stream_t stream) {
@@ -612,6 +673,31 @@ int dsalt_silu_mul(const dsalt_silu_mul_args* a, dsalt_stream_t stream) {
     p.out = a->out;
     p.out_st = a->out_stride;
     return hip_status(dsalt::silu_mul_launch(p, (hipStream_t)stream), "dsalt_silu_mul");
+}
+
+int dsalt_sort_landmarks(const dsalt_sort_args* a, dsalt_stream_t stream) {
+    if (!a) return fail(DSALT_ERR_INVALID, "null argument struct");
+    if (a->n_sets < 0 || a->k < 0 || a->k > dsalt::kMaxLandmarks)
+        return fail(DSALT_ERR_INVALID, "n_sets >= 0 and k in [0, %d] required (got %lld, %d)", dsalt::kMaxLandmarks,
+                    (long long)a->n_sets, a->k);
+    if (a->idx_bytes != 4 && a->idx_bytes != 8)
+        return fail(DSALT_ERR_INVALID, "idx_bytes must be 4 or 8, got %d", a->idx_bytes);
+    if (a->n_sets == 0 || a->k == 0) return DSALT_OK;
+    if (!a->idx || !a->sorted || !a->perm) return fail(DSALT_ERR_INVALID, "idx, sorted and perm are required");
+    if ((a->bias != nullptr) != (a->bias_sorted != nullptr) ||
+        (a->bias && a->bias_bytes != 2 && a->bias_bytes != 4))
+        return fail(DSALT_ERR_INVALID, "bias and bias_sorted go together, of 2 or 4 bytes an element");
+    dsalt::SortSetsParams p;
+    p.n_sets = a->n_sets;
+    p.k = a->k;
+    p.idx64 = a->idx_bytes == 8;
+    p.idx = a->idx;
+    p.out = a->sorted;
+    p.perm = a->perm;
+    p.bias = a->bias;
+    p.bias_out = a->bias_sorted;
+    p.bias_bytes = a->bias ? a->bias_bytes : 0;
+    return hip_status(dsalt::sort_sets_launch(p, (hipStream_t)stream), "dsalt_sort_landmarks");
 }
 
 int dsalt_gather_landmarks(const dsalt_gather_args* a, dsalt_stream_t stream) {

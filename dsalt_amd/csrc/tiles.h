@@ -145,6 +145,22 @@ __device__ __forceinline__ void row_op32(const float* lds, int rs, int row, int 
     }
 }
 
+// A float32 row rounded to T in operand layout, and written to dst (both at the row's start;
+// nullptr: zeros, nothing written).
+template <typename T, int D>
+__device__ __forceinline__ void load_rounded(typename Vec8<T>::type (&x)[D / 32], const float* src, const float* any_valid,
+                                             T* dst, int g) {
+    const float* p = src ? src : any_valid;
+#pragma unroll
+    for (int dc = 0; dc < D / 32; ++dc) {
+        const floatx4 a = *(const floatx4*)(p + dc * 32 + 8 * g), b = *(const floatx4*)(p + dc * 32 + 8 * g + 4);
+        typename Vec8<T>::type v = pack8<T>(a, b);
+        if (!src) v = typename Vec8<T>::type{};
+        else *(typename Vec8<T>::type*)(dst + dc * 32 + 8 * g) = v;
+        x[dc] = v;
+    }
+}
+
 // Register copy of one token row in operand layout (queries in the forward
 // and dq kernels, keys/values in the key-parallel kernels).
 template <typename T, int D>
@@ -313,13 +329,20 @@ __device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirs
 // D * sizeof(T) / 16 lanes per row, so each store instruction writes whole rows (stores of
 // 8-byte pieces, four instructions per row, cost the kernels up to a tenth of their time).
 // dst(rr) is row rr's destination (rr = 0..15, the row of accumulator lane rr), nullptr for
-// a row not written.  Every lane of the wave calls it.
+// a row not written; dst32(rr) likewise where the rounded values go as float32 too (16-bit
+// types: what a caller that wants float32 would convert in a pass of its own).  Every lane of
+// the wave calls it.
 template <typename T, int D>
 struct StoreRows {
     static constexpr int RS = D + 16 / (int)sizeof(T);  // row stride in LDS: 16 bytes of padding
     static constexpr int ELEMS = 16 * RS;
     template <typename Dst>
     __device__ __forceinline__ static void run(T* stage, const floatx4 (&acc)[D / 16], float mul, int lane, Dst dst) {
+        run(stage, acc, mul, lane, dst, [](int) { return (float*)nullptr; });
+    }
+    template <typename Dst, typename Dst32>
+    __device__ __forceinline__ static void run(T* stage, const floatx4 (&acc)[D / 16], float mul, int lane, Dst dst,
+                                               Dst32 dst32) {
         const int j = lane & 15, g = lane >> 4;
 #pragma unroll
         for (int dt = 0; dt < D / 16; ++dt) {
@@ -343,6 +366,14 @@ struct StoreRows {
             const uint4 val = *(const uint4*)(stage + rr * RS + c);
             T* d = dst(rr);
             if (d) *(uint4*)(d + c) = val;
+            if constexpr (sizeof(T) == 2) {
+                float* d32 = dst32(rr);
+                if (d32) {
+                    const T* e = (const T*)&val;
+                    *(floatx4*)(d32 + c) = floatx4{to_float(e[0]), to_float(e[1]), to_float(e[2]), to_float(e[3])};
+                    *(floatx4*)(d32 + c + 4) = floatx4{to_float(e[4]), to_float(e[5]), to_float(e[6]), to_float(e[7])};
+                }
+            }
         }
     }
 };

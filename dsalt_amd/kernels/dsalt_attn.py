@@ -46,6 +46,11 @@ def pad_head_dim(t: torch.Tensor, dp: int) -> torch.Tensor:
     return t if d == dp else torch.nn.functional.pad(t, (0, dp - d))
 
 
+def _direct_f32(q: torch.Tensor, head_dim: int) -> bool:
+    """The forward kernel writes the float32 result itself: 16-bit tensors of a compiled head_dim."""
+    return q.dtype != torch.float32 and q.shape[-1] == head_dim and q.shape[0] > 0
+
+
 class DSALTAttentionFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, q, k, v, lmk_indices, lmk_bias, w_sizes, cu_seqlens, max_seqlen=None, block_size=512):
@@ -65,14 +70,19 @@ class DSALTAttentionFunction(torch.autograd.Function):
         q, k, v = (pad_head_dim(t, dp) for t in (q, k, v))
         plan = ops.new_plan(q, k, cu_i, idx_s, max_seqlen=max_seqlen, select_mode=mode, block_size=block_size)
         variant = tuned_variant(dp, q.device, q.dtype)  # autotune_blocks' choice, if made
+        # the float32 result comes from the kernel itself (the rounded values stay for the backward)
+        out32 = torch.empty(q.shape, dtype=torch.float32, device=q.device) if _direct_f32(q, head_dim) else None
         out, lse = ops.attention_forward(q, k, v, w_i, cu_i, idx_s, bias_s, scale=scale, max_seqlen=max_seqlen,
-                                         select_mode=mode, block_size=block_size, plan=plan, variant=variant)
+                                         select_mode=mode, block_size=block_size, plan=plan, variant=variant,
+                                         out_f32=out32)
         ctx.save_for_backward(q, k, v, out, lse, idx_s, bias_s if bias_s is not None else torch.empty(0),
                               perm, w_i, cu_i, plan)
         ctx.has_bias = bias_s is not None
         ctx.mode, ctx.max_seqlen, ctx.scale, ctx.variant = mode, max_seqlen, scale, variant
         ctx.bias_dtype = lmk_bias.dtype if lmk_bias is not None else None
         ctx.head_dim = head_dim
+        if out32 is not None:
+            return out32
         return out[..., :head_dim].float().contiguous()
 
     @staticmethod
@@ -80,14 +90,14 @@ class DSALTAttentionFunction(torch.autograd.Function):
         q, k, v, out, lse, idx_s, bias_s, perm, w_i, cu_i, plan = ctx.saved_tensors
         if ctx.mode == ops.SELECT_BLOCK:
             raise NotImplementedError("the backward of the block-causal landmark variant is not implemented")
-        go = pad_head_dim(grad_out.to(q.dtype), q.shape[-1])
+        go = grad_out if ctx.head_dim == q.shape[-1] else pad_head_dim(grad_out.to(q.dtype), q.shape[-1])
         dq, dk, dv, db = ops.attention_backward(go, q, k, v, out, lse, w_i, cu_i, idx_s,
                                                 bias_s if ctx.has_bias else None, scale=ctx.scale,
                                                 max_seqlen=ctx.max_seqlen, want_dbias=ctx.needs_input_grad[4],
                                                 plan=plan, variant=ctx.variant)
         d_bias = None
         if ctx.needs_input_grad[4] and db is not None:
-            d_bias = torch.zeros_like(db).scatter_(-1, perm, db)[:, :, 0].to(ctx.bias_dtype)
+            d_bias = torch.empty_like(db).scatter_(-1, perm, db)[:, :, 0].to(ctx.bias_dtype)
         d = ctx.head_dim
         if d != q.shape[-1]:
             dq, dk, dv = (t[..., :d].contiguous() for t in (dq, dk, dv))

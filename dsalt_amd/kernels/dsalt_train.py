@@ -31,7 +31,7 @@ import torch
 
 from .. import ops
 from .autotune import tuned_variant
-from .dsalt_attn import pad_head_dim, padded_head_dim
+from .dsalt_attn import _direct_f32, pad_head_dim, padded_head_dim
 
 
 class DSALTTrainFunction(torch.autograd.Function):
@@ -50,27 +50,30 @@ class DSALTTrainFunction(torch.autograd.Function):
         q, k, v = (pad_head_dim(t, dp) for t in (q, k, v))
         plan = ops.new_plan(q, k, cu_i, idx_s, max_seqlen=max_seqlen)
         variant = tuned_variant(dp, q.device, q.dtype)  # autotune_blocks' choice, if made
+        out32 = torch.empty(q.shape, dtype=torch.float32, device=q.device) if _direct_f32(q, head_dim) else None
         out, lse = ops.train_forward(q, k, v, w_c, cu_i, idx_s, logw_s, tau_win=float(tau_win),
                                      win_edge=float(win_edge), scale=scale, max_seqlen=max_seqlen, plan=plan,
-                                     variant=variant)
+                                     variant=variant, out_f32=out32)
         ctx.save_for_backward(q, k, v, out, lse, idx_s, logw_s, perm, w_c, cu_i, plan)
         ctx.max_seqlen, ctx.scale, ctx.variant = max_seqlen, scale, variant
         ctx.tau_win, ctx.win_edge = float(tau_win), float(win_edge)
         ctx.logw_dtype, ctx.w_dtype = lmk_logw.dtype, w_cont.dtype
         ctx.head_dim = head_dim
+        if out32 is not None:
+            return out32
         return out[..., :head_dim].float().contiguous()
 
     @staticmethod
     def backward(ctx, grad_out):
         q, k, v, out, lse, idx_s, logw_s, perm, w_c, cu_i, plan = ctx.saved_tensors
         dq, dk, dv, dlogw, d_w = ops.train_backward(
-            pad_head_dim(grad_out.to(q.dtype), q.shape[-1]), q, k, v, out, lse, w_c, cu_i, idx_s, logw_s,
+            grad_out if ctx.head_dim == q.shape[-1] else pad_head_dim(grad_out.to(q.dtype), q.shape[-1]), q, k, v, out, lse, w_c, cu_i, idx_s, logw_s,
             tau_win=ctx.tau_win,
             win_edge=ctx.win_edge, scale=ctx.scale, max_seqlen=ctx.max_seqlen,
             want_dlogw=ctx.needs_input_grad[4], plan=plan, variant=ctx.variant)
         d_logw = None
         if ctx.needs_input_grad[4] and dlogw is not None:
-            d_logw = torch.zeros_like(dlogw).scatter_(-1, perm, dlogw)[:, :, 0].to(ctx.logw_dtype)
+            d_logw = torch.empty_like(dlogw).scatter_(-1, perm, dlogw)[:, :, 0].to(ctx.logw_dtype)
         d_wc = d_w.to(ctx.w_dtype) if ctx.needs_input_grad[5] else None
         d = ctx.head_dim
         if d != q.shape[-1]:

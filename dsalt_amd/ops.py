@@ -15,7 +15,7 @@ from . import _lib
 from ._lib import (DTYPE_BF16, DTYPE_F16, DTYPE_F32, SELECT_BLOCK, SELECT_GLOBAL, STATS_PACKED,
                    STATS_SEQUENCE, VARIANT_DEFAULT, VARIANT_DQ_BN64, VARIANT_FWD_BN32, VARIANT_FWD_RG2,
                    VARIANT_LMK_SHORT, BwdArgs, CeArgs, FwdArgs, GatherArgs, Problem, ProbsArgs, RopeArgs, SelectArgs,
-                   SiluMulArgs,
+                   SiluMulArgs, SortArgs,
                    TrainBwdArgs,
                    TrainFwdArgs)
 
@@ -248,13 +248,14 @@ def _check_plan(plan, a) -> int:
 
 def attention_forward(q, k, v, w, cu_seqlens, lmk_idx, lmk_bias=None, *, scale=None,
                       max_seqlen=None, select_mode=SELECT_GLOBAL, block_size=512, plan=None,
-                      variant=VARIANT_DEFAULT, plan_ready=False):
+                      variant=VARIANT_DEFAULT, plan_ready=False, out_f32=None):
     """(out [T,H,D] in q.dtype, lse [T,H] fp32).  lmk_idx [H,S,n_sets,K] int32 ascending with
     -1 padding at the end of each set (as select_landmarks returns; a position may repeat, each
     copy counts).  ``plan`` (ops.new_plan) receives the row plan for attention_backward of the
     same rows; ``variant`` picks a tiling (VARIANT_* bits, kernels.autotune); ``plan_ready``:
     ``plan`` already holds the row plan of these windows (select_landmarks(plan=...)), so the
-    forward reads it instead of recomputing it."""
+    forward reads it instead of recomputing it; ``out_f32`` (contiguous float32 [T,H,D], with
+    16-bit tensors) receives the rounded outputs as float32 too."""
     a, out, lse, keep = _fwd_args(q, k, v, w, cu_seqlens, lmk_idx, lmk_bias, scale, max_seqlen, select_mode,
                                   block_size)
     a.plan = _check_plan(plan, a) or None
@@ -265,8 +266,18 @@ def attention_forward(q, k, v, w, cu_seqlens, lmk_idx, lmk_bias=None, *, scale=N
     dev = out.device
     L = _lib.load()
     ws = _set_workspace(a, L.dsalt_fwd_workspace_bytes(ctypes.byref(a)), dev)  # noqa: F841 (kept alive)
-    _lib.check("dsalt_fwd", L.dsalt_fwd(ctypes.byref(a), _stream(dev)))
+    if out_f32 is not None:
+        _check_out_f32(out_f32, out)
+        _lib.check("dsalt_fwd", L.dsalt_fwd_f32out(ctypes.byref(a), _ptr(out_f32), _stream(dev)))
+    else:
+        _lib.check("dsalt_fwd", L.dsalt_fwd(ctypes.byref(a), _stream(dev)))
     return out, lse
+
+
+def _check_out_f32(t: torch.Tensor, out: torch.Tensor):
+    if t.dtype != torch.float32 or t.shape != out.shape or not t.is_contiguous() or t.device != out.device \
+            or out.dtype == torch.float32:
+        raise ValueError("out_f32 must be a contiguous float32 tensor of the 16-bit output's shape")
 
 
 def _w_cont(w_cont: torch.Tensor, T: int) -> torch.Tensor:
@@ -276,10 +287,10 @@ def _w_cont(w_cont: torch.Tensor, T: int) -> torch.Tensor:
 
 
 def train_forward(q, k, v, w_cont, cu_seqlens, lmk_idx, lmk_logw, *, tau_win=1.0, win_edge=4.0, scale=None,
-                  max_seqlen=None, plan=None, variant=VARIANT_DEFAULT):
+                  max_seqlen=None, plan=None, variant=VARIANT_DEFAULT, out_f32=None):
     """Training variant: (out [T,H,D] in q.dtype, lse [T,H] fp32).  w_cont [T] continuous
     windows; lmk_idx [H,S,1,K] ascending with -1 last; lmk_logw [H,S,1,K] landmark log-weights
-    (-inf or any value in -1 slots)."""
+    (-inf or any value in -1 slots).  ``out_f32``: as in attention_forward."""
     a, out, lse, keep = _fwd_args(q, k, v, w_cont, cu_seqlens, lmk_idx, lmk_logw, scale, max_seqlen,
                                   SELECT_GLOBAL, 0, need_w=False)
     a.plan = _check_plan(plan, a) or None
@@ -293,7 +304,11 @@ def train_forward(q, k, v, w_cont, cu_seqlens, lmk_idx, lmk_logw, *, tau_win=1.0
     L = _lib.load()
     ws = _workspace(L.dsalt_train_fwd_workspace_bytes(ctypes.byref(t)), dev)
     t.base.workspace, t.base.workspace_bytes = ws.data_ptr(), ws.numel()
-    _lib.check("dsalt_train_fwd", L.dsalt_train_fwd(ctypes.byref(t), _stream(dev)))
+    if out_f32 is not None:
+        _check_out_f32(out_f32, out)
+        _lib.check("dsalt_train_fwd", L.dsalt_train_fwd_f32out(ctypes.byref(t), _ptr(out_f32), _stream(dev)))
+    else:
+        _lib.check("dsalt_train_fwd", L.dsalt_train_fwd(ctypes.byref(t), _stream(dev)))
     return out, lse
 
 
@@ -305,8 +320,12 @@ def _bwd_args(dout, q, k, v, out, lse, w, cu_seqlens, lmk_idx, lmk_bias, scale, 
     q, k, v, out, dout = (_rows3(t, n) for t, n in ((q, "q"), (k, "k"), (v, "v"), (out, "out"),
                                                    (dout, "dout")))
     dt = dtype_code(q.dtype)
+    d32 = None
     if dout.dtype != q.dtype:
-        dout = dout.to(q.dtype)
+        if _f32_rows(dout, q):  # rounded by the dQ pass into the buffer the later passes read
+            d32, dout = dout, torch.empty(dout.shape, dtype=q.dtype, device=dev)
+        else:
+            dout = dout.to(q.dtype)
     T, H, D = q.shape
     G = k.shape[1]
     S = cu_seqlens.shape[0] - 1
@@ -343,7 +362,15 @@ def _bwd_args(dout, q, k, v, out, lse, w, cu_seqlens, lmk_idx, lmk_bias, scale, 
     a.dq, a.dk, a.dv = dq.data_ptr(), dk.data_ptr(), dv.data_ptr()
     a.d_bias = db.data_ptr() if db is not None and db.numel() else None
     a.scale = scale
-    return a, dq, dk, dv, db, (q, k, v, out, dout, w_c, cu_c, li, lb, lse)
+    return a, dq, dk, dv, db, d32, (q, k, v, out, dout, w_c, cu_c, li, lb, lse)
+
+
+def _f32_rows(t: torch.Tensor, q: torch.Tensor) -> bool:
+    """A float32 upstream gradient the 16-bit kernels round themselves: 16-byte aligned rows with
+    positive token stride."""
+    return (t.dtype == torch.float32 and q.dtype != torch.float32 and t.shape == q.shape and t.stride(2) == 1
+            and t.data_ptr() % 16 == 0 and t.stride(0) > 0 and t.stride(0) % 4 == 0 and t.stride(1) >= 0
+            and t.stride(1) % 4 == 0)
 
 
 def attention_backward(dout, q, k, v, out, lse, w, cu_seqlens, lmk_idx, lmk_bias=None, *,
@@ -352,8 +379,8 @@ def attention_backward(dout, q, k, v, out, lse, w, cu_seqlens, lmk_idx, lmk_bias
     Global selection variant; grouped key/value heads are read in place and their gradients
     summed over the group inside the kernels.  ``plan``: the buffer attention_forward filled
     for the same rows (skips recomputing the row plan)."""
-    a, dq, dk, dv, db, keep = _bwd_args(dout, q, k, v, out, lse, w, cu_seqlens, lmk_idx, lmk_bias, scale,
-                                        max_seqlen, want_dbias)
+    a, dq, dk, dv, db, d32, keep = _bwd_args(dout, q, k, v, out, lse, w, cu_seqlens, lmk_idx, lmk_bias, scale,
+                                             max_seqlen, want_dbias)
     a.plan = _check_plan(plan, a) or None
     a.variant = int(variant)
     if q.shape[0] == 0:
@@ -365,7 +392,11 @@ def attention_backward(dout, q, k, v, out, lse, w, cu_seqlens, lmk_idx, lmk_bias
         _lib.check("dsalt_bwd", L.dsalt_bwd(ctypes.byref(a), None))
     ws = _workspace(need, dev)
     a.workspace, a.workspace_bytes = ws.data_ptr(), ws.numel()
-    _lib.check("dsalt_bwd", L.dsalt_bwd(ctypes.byref(a), _stream(dev)))
+    if d32 is not None:
+        _lib.check("dsalt_bwd", L.dsalt_bwd_f32dout(ctypes.byref(a), _ptr(d32), d32.stride(0), d32.stride(1),
+                                                    _stream(dev)))
+    else:
+        _lib.check("dsalt_bwd", L.dsalt_bwd(ctypes.byref(a), _stream(dev)))
     return dq, dk, dv, db
 
 
@@ -373,8 +404,8 @@ def train_backward(dout, q, k, v, out, lse, w_cont, cu_seqlens, lmk_idx, lmk_log
                    win_edge=4.0, scale=None, max_seqlen=None, want_dlogw=True, plan=None, variant=VARIANT_DEFAULT):
     """Training variant: (dq [T,H,D], dk, dv [T,n_kv,D]) in q.dtype, d_logw [H,S,1,K] fp32 (or
     None) and d_w [T] fp32, the window gradient summed over heads."""
-    a, dq, dk, dv, db, keep = _bwd_args(dout, q, k, v, out, lse, w_cont, cu_seqlens, lmk_idx, lmk_logw, scale,
-                                        max_seqlen, want_dlogw, need_w=False)
+    a, dq, dk, dv, db, d32, keep = _bwd_args(dout, q, k, v, out, lse, w_cont, cu_seqlens, lmk_idx, lmk_logw, scale,
+                                             max_seqlen, want_dlogw, need_w=False)
     a.plan = _check_plan(plan, a) or None
     a.variant = int(variant)
     T = q.shape[0]
@@ -392,7 +423,11 @@ def train_backward(dout, q, k, v, out, lse, w_cont, cu_seqlens, lmk_idx, lmk_log
         _lib.check("dsalt_train_bwd", L.dsalt_train_bwd(ctypes.byref(t), None))
     ws = _workspace(need, dev)
     t.base.workspace, t.base.workspace_bytes = ws.data_ptr(), ws.numel()
-    _lib.check("dsalt_train_bwd", L.dsalt_train_bwd(ctypes.byref(t), _stream(dev)))
+    if d32 is not None:
+        _lib.check("dsalt_train_bwd", L.dsalt_train_bwd_f32dout(ctypes.byref(t), _ptr(d32), d32.stride(0), d32.stride(1),
+                                                                _stream(dev)))
+    else:
+        _lib.check("dsalt_train_bwd", L.dsalt_train_bwd(ctypes.byref(t), _stream(dev)))
     return dq, dk, dv, db, d_w
 
 
@@ -606,6 +641,25 @@ def silu_mul(gate: torch.Tensor, up: torch.Tensor, out: torch.Tensor | None = No
 def sort_landmarks(idx: torch.Tensor, bias: torch.Tensor | None = None):
     """Sort each set ascending with -1 last (the order the kernels require); returns
     (sorted int32 indices, bias permuted the same way or None, permutation)."""
+    b_ok = bias is None or (bias.element_size() in (2, 4) and bias.device == idx.device and bias.shape == idx.shape
+                            and not (torch.is_grad_enabled() and bias.requires_grad))
+    if idx.device.type == "cuda" and idx.dtype in (torch.int32, torch.int64) and b_ok \
+            and 0 < idx.shape[-1] <= MAX_LANDMARKS and idx.numel():
+        src = idx.detach().contiguous()
+        out = torch.empty(src.shape, dtype=torch.int32, device=src.device)
+        perm = torch.empty(src.shape, dtype=torch.int64, device=src.device)
+        a = SortArgs()
+        a.k = src.shape[-1]
+        a.n_sets, a.idx_bytes = src.numel() // a.k, src.element_size()
+        a.idx, a.sorted, a.perm = src.data_ptr(), out.data_ptr(), perm.data_ptr()
+        b = None
+        if bias is not None:
+            bc = bias.detach().contiguous()
+            b = torch.empty_like(bc)
+            a.bias, a.bias_sorted, a.bias_bytes = bc.data_ptr(), b.data_ptr(), bc.element_size()
+        L = _lib.load()
+        _lib.check("dsalt_sort_landmarks", L.dsalt_sort_landmarks(ctypes.byref(a), _stream(src.device)))
+        return out, b, perm
     big = torch.iinfo(torch.int32).max
     key = torch.where(idx < 0, torch.full_like(idx, big), idx).to(torch.int64)
     srt, perm = key.sort(dim=-1)

@@ -314,6 +314,24 @@ typedef struct dsalt_silu_mul_args {
 
 int    dsalt_silu_mul(const dsalt_silu_mul_args* a, dsalt_stream_t stream);
 
+/* Landmark sets in any order put into the one dsalt_fwd / dsalt_bwd take: positions
+ * ascending, empty slots (any negative value) as -1 at the end; equal positions keep their
+ * order.  perm is the source slot of each output slot; bias (optional) follows the same
+ * order.  Contiguous [n_sets, k] arrays. */
+typedef struct dsalt_sort_args {
+    int64_t n_sets;
+    int32_t k;                 /* 0..2048                                            */
+    int32_t idx_bytes;         /* 4 (int32) or 8 (int64)                             */
+    const void* idx;
+    int32_t* sorted;
+    int64_t* perm;
+    const void* bias;          /* NULL, or elements of bias_bytes (2 or 4) bytes     */
+    void* bias_sorted;
+    int32_t bias_bytes;
+} dsalt_sort_args;
+
+int    dsalt_sort_landmarks(const dsalt_sort_args* a, dsalt_stream_t stream);
+
 /* Tile variants of the attention kernels (dsalt_fwd_args.variant, dsalt_bwd_args.variant).
  * Bits are independent; a bit a shape cannot use is ignored.  Without forward bits the
  * operator's forward picks its tiling by the call's size (attn_fwd.hip::fwd_variant). */
@@ -338,6 +356,9 @@ int    dsalt_select(const dsalt_select_args* a, dsalt_stream_t stream);
 /* Workspace of dsalt_fwd: the row plan, or 0 when a->plan supplies it. */
 size_t dsalt_fwd_workspace_bytes(const dsalt_fwd_args* a);
 int    dsalt_fwd(const dsalt_fwd_args* a, dsalt_stream_t stream);
+/* dsalt_fwd that also writes the rounded outputs as float32, contiguous [T, H, D] (16-bit
+ * tensors; `out` is written as well, for the backward). */
+int    dsalt_fwd_f32out(const dsalt_fwd_args* a, float* out_f32, dsalt_stream_t stream);
 
 /* dsalt_fwd without allocations or a workspace argument.  No counterpart in the
  * reference: it is for callers that cannot allocate device memory (code under HIP
@@ -359,13 +380,20 @@ int    dsalt_fwd_noalloc(const dsalt_fwd_args* a, dsalt_stream_t stream);
  * a->plan supplies it). */
 size_t dsalt_bwd_workspace_bytes(const dsalt_bwd_args* a);
 int    dsalt_bwd(const dsalt_bwd_args* a, dsalt_stream_t stream);
+/* dsalt_bwd of an upstream gradient in float32 (16-bit tensors; strides in elements,
+ * multiples of four): its values rounded to the tensor type are used, and written to `dout`. */
+int    dsalt_bwd_f32dout(const dsalt_bwd_args* a, const float* dout_f32, int64_t stride_t, int64_t stride_h,
+                         dsalt_stream_t stream);
 
 int    dsalt_gather_landmarks(const dsalt_gather_args* a, dsalt_stream_t stream);
 
 size_t dsalt_train_fwd_workspace_bytes(const dsalt_train_fwd_args* a);
 int    dsalt_train_fwd(const dsalt_train_fwd_args* a, dsalt_stream_t stream);
+int    dsalt_train_fwd_f32out(const dsalt_train_fwd_args* a, float* out_f32, dsalt_stream_t stream);
 size_t dsalt_train_bwd_workspace_bytes(const dsalt_train_bwd_args* a);
 int    dsalt_train_bwd(const dsalt_train_bwd_args* a, dsalt_stream_t stream);
+int    dsalt_train_bwd_f32dout(const dsalt_train_bwd_args* a, const float* dout_f32, int64_t stride_t,
+                               int64_t stride_h, dsalt_stream_t stream);
 
 /* Testing hook with no counterpart in the reference: dsalt_select with its
  * top-k working sets shrunk by `border_cap` so tests can drive the paths that
