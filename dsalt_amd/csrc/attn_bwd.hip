@@ -514,11 +514,16 @@ struct QLoader {
 // rows with lo_i > j0 + 63 are skipped.  List order is row order, so the sum
 // order is fixed and results are deterministic.
 // four waves per SIMD for 16-bit head_dim 64 (32-row stages keep it free of spills; three with
-// grouped heads or the training variant, which need more registers), two otherwise.
+// the head loop of grouped heads, which needs more registers), two otherwise.
 // TR: training variant -- fully visible rows must also see every key of the block
 // past their edge_keys edge-bias keys; other rows add the soft edge bias.
 // GQA: the key/value head has several query heads (swept in order); without it the
 // sweep is straight-line code for one head.
+// NH > 1: the block takes the NH query heads of its key/value head at once, one group of four
+// waves and one copy of the staging buffers a head (the windows, and so the row lists, chunks and
+// barriers, are the same for every head), and adds the groups' sums in head order through LDS.
+// Each group runs the one-head code (126 VGPRs, four waves per SIMD, where the head loop holds
+// 159 and three), and a small batch fills the chip instead of walking the heads one after the other.
 template <typename T, int D, int BQ, int NT = 256>
 struct QTiles {  // one staged chunk of the dK/dV sweep: BQ rows of Q and of dO
     typedef Tile<T, D, BQ, NT> QT;
@@ -526,41 +531,61 @@ struct QTiles {  // one staged chunk of the dK/dV sweep: BQ rows of Q and of dO
     T d[QT::ELEMS];
 };
 
-template <typename T, int D, bool TR, bool GQA>
-__global__ __launch_bounds__(256, (sizeof(T) == 2 && D == 64) ? ((GQA || TR) ? 3 : 4) : 2) void bwd_dkdv_kernel(AttnParams p) {
-    constexpr int BQ = BwdShape<T, D>::BQ;
-    constexpr int NQS = BQ / 16;
-    constexpr int NDIAG = 64 / BQ;
-    constexpr bool kHalf = sizeof(T) == 2;
+template <typename T, int D, bool TR>
+struct DkdvShared {
+    static constexpr int BQ = BwdShape<T, D>::BQ;
     // list positions of a segment: full rows from 0, partial rows from the next chunk
     // boundary, each list padded to whole chunks
-    constexpr int kLst = kSeg + 2 * BQ;
-    typedef QTiles<T, D, BQ> QS;
-    typedef typename QS::QT QT;
-    __shared__ __attribute__((aligned(16))) QS sq[2];
-    __shared__ int wcnt[4][8];
+    static constexpr int kLst = kSeg + 2 * BQ;
+    __attribute__((aligned(16))) QTiles<T, D, BQ> sq[2];
     // per-row data of the rows a chunk covers, in chunk order, read by the products straight
     // from these tables: window start (0x7fffffff for no row), LSE in base 2, -delta (0 for
     // no row)[, continuous window, row index]; a segment's rows in list order with their row
     // offsets (-1 for padding) for the gathers, the 64 diagonal rows in row order
-    __shared__ short lrw[kLst];
-    __shared__ __attribute__((aligned(16))) int lt_lo[kLst];
-    __shared__ __attribute__((aligned(16))) float lt_l[kLst], lt_d[kLst];
-    __shared__ __attribute__((aligned(16))) float lt_wt[TR ? kLst : 4];
-    __shared__ __attribute__((aligned(16))) int lt_ri[TR ? kLst : 4];
-    __shared__ __attribute__((aligned(16))) int dt_lo[64];
-    __shared__ __attribute__((aligned(16))) float dt_l[64], dt_d[64];
-    __shared__ __attribute__((aligned(16))) float dt_wt[TR ? 64 : 4];
-    __shared__ int own_s[64];  // per key of the block: h * K + slot of its owner, or kNoOwner
-    __shared__ int wmax_s[4];
+    __attribute__((aligned(16))) int lt_lo[kLst];
+    __attribute__((aligned(16))) float lt_l[kLst], lt_d[kLst];
+    __attribute__((aligned(16))) float lt_wt[TR ? kLst : 4];
+    __attribute__((aligned(16))) int lt_ri[TR ? kLst : 4];
+    __attribute__((aligned(16))) int dt_lo[64];
+    __attribute__((aligned(16))) float dt_l[64], dt_d[64];
+    __attribute__((aligned(16))) float dt_wt[TR ? 64 : 4];
+    short lrw[kLst];
+    int wcnt[4][8];
+    int wmax_s[4];
+};
 
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, g = lane >> 4;
+template <typename T, int D, bool TR, bool GQA, int NH = 1>
+__global__ __launch_bounds__(256 * NH, (sizeof(T) == 2 && D == 64) ? (GQA ? 3 : 4) : 2) void bwd_dkdv_kernel(AttnParams p) {
+    static_assert(NH == 1 || !GQA, "heads side by side: one head per group of waves");
+    constexpr int BQ = BwdShape<T, D>::BQ;
+    constexpr int NQS = BQ / 16;
+    constexpr int NDIAG = 64 / BQ;
+    constexpr bool kHalf = sizeof(T) == 2;
+    typedef QTiles<T, D, BQ> QS;
+    typedef typename QS::QT QT;
+    __shared__ DkdvShared<T, D, TR> shm[NH];
+    __shared__ int own_s[64];  // per key of the block: h * K + slot of its owner, or kNoOwner
+    // the group of four waves (one query head each), its buffers, and the thread within it
+    const int grp = NH > 1 ? uniform((int)threadIdx.x >> 8) : 0;
+    auto& sm = shm[grp];
+    auto& sq = sm.sq;
+    auto &lrw = sm.lrw;
+    int *const lt_lo = sm.lt_lo, *const dt_lo = sm.dt_lo;
+    float *const lt_l = sm.lt_l, *const lt_d = sm.lt_d, *const dt_l = sm.dt_l, *const dt_d = sm.dt_d;
+    float *const lt_wt = sm.lt_wt, *const dt_wt = sm.dt_wt;
+    int* const lt_ri = sm.lt_ri;
+    auto& wcnt = sm.wcnt;
+    auto& wmax_s = sm.wmax_s;
+
+    const int tid = NH > 1 ? (int)threadIdx.x & 255 : (int)threadIdx.x;
+    const int wave = tid >> 6, lane = tid & 63, g = lane >> 4;
     const int total = p.n_kv_heads * p.num_seqs * p.n_tiles;
     const int L = xcd_swizzle(blockIdx.x, total);
     const int t = L % p.n_tiles;
     const int s = (L / p.n_tiles) % p.num_seqs;
     const int kvh = L / (p.n_tiles * p.num_seqs);
-    const int rep = GQA ? p.n_heads / p.n_kv_heads : 1;
+    const int rep = GQA ? p.n_heads / p.n_kv_heads : 1;  // heads this group of waves sweeps
+    const int h0 = NH > 1 ? kvh * NH + grp : kvh * rep;  // the first of them
     int st, len;
     seq_bounds(p.cu, s, p.total_len, p.max_seqlen, st, len);
     const int j0 = t * 64;
@@ -602,7 +627,7 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 && D == 64) ? ((GQA || TR) ? 3
     // the query heads of this key/value head are swept one after the other (head order),
     // all adding into the same dK/dV registers
     for (int hh = 0; hh < rep; ++hh) {
-    const int h = kvh * rep + hh;
+    const int h = h0 + hh;
     const T* qb = (const T*)p.q + (int64_t)st * p.q_st + (int64_t)h * p.q_sh;
     const T* db = (const T*)p.dout + (int64_t)st * p.do_st + (int64_t)h * p.do_sh;
     const float* lrow = p.lse2t + (int64_t)h * p.total_len + st;
@@ -798,7 +823,7 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 && D == 64) ? ((GQA || TR) ? 3
     int ov = -1, ovp = -1;  // this thread's landmark slot among the first 256 of the group, and the one before
     const int K = p.k_lmk;
     const int nown = rep * K;
-    const int32_t* oset = p.lmk + (((int64_t)(kvh * rep + min(tid, max(nown, 1) - 1) / max(K, 1)) * p.num_seqs + s) *
+    const int32_t* oset = p.lmk + (((int64_t)(h0 + min(tid, max(nown, 1) - 1) / max(K, 1)) * p.num_seqs + s) *
                                    p.n_sets) * K;
     const int osl = K > 0 ? min(tid, nown - 1) % K : 0;
     if (hh == 0) {
@@ -829,7 +854,7 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 && D == 64) ? ((GQA || TR) ? 3
     if (kPre) count_rows(bf, bp);
     int own_at = -1, own_id = 0;
     if (hh == 0) {
-        if (tid < 64) own_s[tid] = kNoOwner;
+        if (grp == 0 && tid < 64) own_s[tid] = kNoOwner;
         int wm = 1;
 #pragma unroll
         for (int k = 0; k < kWm; ++k) wm = max(wm, wmv[k]);
@@ -840,7 +865,7 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 && D == 64) ? ((GQA || TR) ? 3
         asm volatile("" : "+v"(ov), "+v"(ovp));
         if (tid < nown && ov >= j0 && ov < dend && (osl == 0 || ovp != ov)) {
             own_at = ov - j0;
-            own_id = (kvh * rep + tid / K) * K + osl;
+            own_id = (h0 + tid / K) * K + osl;
         }
     }
     __syncthreads();
@@ -849,9 +874,9 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 && D == 64) ? ((GQA || TR) ? 3
         if (own_at >= 0) atomicMin(own_s + own_at, own_id);
         for (int e = tid + 256; e < rep * K; e += 256) {  // groups of more than 256 slots
             const int hs = e / K, sl = e % K;
-            const int32_t* set = p.lmk + (((int64_t)(kvh * rep + hs) * p.num_seqs + s) * p.n_sets) * K;
+            const int32_t* set = p.lmk + (((int64_t)(h0 + hs) * p.num_seqs + s) * p.n_sets) * K;
             const int v = set[sl];
-            if (v >= j0 && v < dend && (sl == 0 || set[sl - 1] != v)) atomicMin(own_s + (v - j0), (kvh * rep + hs) * K + sl);
+            if (v >= j0 && v < dend && (sl == 0 || set[sl - 1] != v)) atomicMin(own_s + (v - j0), (h0 + hs) * K + sl);
         }
     }
     if (kPre) list_rows(bf, bp, [&](int u) { return rdat[u]; }, seg0);
@@ -921,6 +946,30 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 && D == 64) ? ((GQA || TR) ? 3
         }
     }
     }  // query heads of the group
+
+    if constexpr (NH > 1) {
+        // the groups' sums, added in head order by group 0: dK, then dV through the tile buffers
+        // (idle after the last barrier), a wave's accumulators as whole 16-byte lanes
+        static_assert(sizeof(sq) >= sizeof(floatx4) * 256 * (D / 16), "a group's sums do not fit its tile buffers");
+        auto merge = [&](floatx4 (&acc)[D / 16]) {
+            floatx4* mine = (floatx4*)&sq[0] + wave * 64 * (D / 16) + lane;
+            if (grp > 0)
+#pragma unroll
+                for (int dt = 0; dt < D / 16; ++dt) mine[dt * 64] = acc[dt];
+            __syncthreads();
+            if (grp == 0)
+#pragma unroll
+                for (int u = 1; u < NH; ++u) {
+                    const floatx4* o = (const floatx4*)&shm[u].sq[0] + wave * 64 * (D / 16) + lane;
+#pragma unroll
+                    for (int dt = 0; dt < D / 16; ++dt) acc[dt] += o[dt * 64];
+                }
+        };
+        merge(adk);
+        __syncthreads();
+        merge(adv);
+        if (grp > 0) return;
+    }
 
     bool owner = false;
     if (jvalid && p.k_lmk > 0) {
@@ -1155,80 +1204,172 @@ __device__ __forceinline__ int find_slot(const int32_t* set, int K, int pos) {
     return lo < K && set[lo] == pos ? lo : -1;
 }
 
-// One thread per (head, sequence, slot, column): d_bias from the slot's chunk partials in
-// chunk order; the owner of a landmark row (the first (head, slot) of the key/value head's
-// group holding it) writes the row's dK/dV once: its band sums from the dK/dV pass, then
-// the chunk partials of every head of the group holding the row, heads and chunks in
-// order, rounded to the output type once.
-template <typename T, int D>
+// WPR waves per (head, sequence, slot), D / 64 columns per lane, each taking a contiguous part of
+// the chunk partials; the owner of a landmark row (the first (head, slot) of the key/value head's
+// group holding it) writes the row's dK/dV once, rounded to the output type once: its band sums
+// from the dK/dV pass plus the partials of every head of the group holding the row, chunks in order
+// within a head, heads in order, then the waves' sums in order (no order depends on the
+// schedule).  d_bias adds the slot's own partials in chunk order.
+// The kernel is a chain of dependent loads, not bandwidth: grouped heads share their value norms,
+// so their sets mostly agree and one owner sums every head's partials.  Sets of up to 128 slots are
+// therefore searched by the whole wave (a binary search is seven dependent loads a head), four
+// heads' sets and then partials in flight at a time, and four waves share a row of at least
+// kSumSplit chunks while the rows with sums to add (about rows / heads of a group) are fewer than
+// kSumFill, two waves per SIMD; from there on one wave a row keeps the memory busy (2048 owners of
+// 32 chunks: 9.9 us with one wave a row, 13.0 with four; 512 owners of 16 chunks: 11.5 and 7.0).  16/4 heads x 8192, head_dim 128: 26.6 -> 13.8 us; 8/2 heads, 5 short sequences: 13.9 -> 7.2.
+constexpr int kSumSplit = 8, kSumFill = 2048;
+
+template <typename T, int D, int WPR>
 __global__ __launch_bounds__(256) void bwd_lmk_sum_kernel(AttnParams p) {
-    const int K = p.k_lmk;
-    const int64_t nrow = (int64_t)p.n_heads * p.num_seqs * K;
-    const int64_t id = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (id >= nrow * D) return;
-    const int d = (int)(id % D);
-    const int64_t row = id / D;  // (h, s, slot)
+    constexpr int CPL = D / 64;  // columns per lane
+    typedef float vec __attribute__((ext_vector_type(CPL)));
+    __shared__ __attribute__((aligned(16))) vec red[WPR > 1 ? 2 * 4 * 64 : 1];
+    const int K = p.k_lmk, lane = threadIdx.x & 63, wave = uniform((int)threadIdx.x >> 6);
+    const int64_t row = WPR > 1 ? (int64_t)blockIdx.x : (int64_t)blockIdx.x * 4 + wave;  // (h, s, slot)
+    const int part = WPR > 1 ? wave : 0;
+    if (row >= (int64_t)p.n_heads * p.num_seqs * K) return;
     const int sl = (int)(row % K);
     const int s = (int)((row / K) % p.num_seqs);
     const int h = (int)(row / ((int64_t)K * p.num_seqs));
-    const int rep = p.n_heads / p.n_kv_heads, kvh = h / rep;
-    const int32_t* set = p.lmk + (((int64_t)h * p.num_seqs + s) * p.n_sets) * K;
-    const int pos = set[sl];
+    const int rep = p.n_heads / p.n_kv_heads, kvh = h / rep, hend = (kvh + 1) * rep;
+    auto set_of = [&](int hh) { return p.lmk + (((int64_t)hh * p.num_seqs + s) * p.n_sets) * K; };
+    // the first batch of sets and the band sums are requested with the position: one latency
+    constexpr int HB = 4;
+    const bool wide = K > 128;
+    int v0[HB], v1[HB];
+    auto load_sets = [&](int hb) {
+#pragma unroll
+        for (int u = 0; u < HB; ++u) {
+            const int32_t* set = set_of(min(hb + u, hend - 1));
+            v0[u] = set[min(lane, K - 1)];
+            v1[u] = set[min(64 + lane, K - 1)];
+        }
+    };
+    if (!wide) load_sets(kvh * rep);
+    const int pos = set_of(h)[sl];
+    const int64_t half = (int64_t)p.n_heads * p.num_seqs * K * D;
+    const int64_t so = row * D + lane * CPL;
+    vec sk = *(const vec*)(p.lmk_stage + so), sv = *(const vec*)(p.lmk_stage + half + so);
     int st, len;
     seq_bounds(p.cu, s, p.total_len, p.max_seqlen, st, len);
     const int64_t cstride = (int64_t)p.n_heads * p.num_seqs * K;
-    auto prow = [&](int hh, int slot) { return (int64_t)hh * p.num_seqs * K + (int64_t)s * K + slot; };
-    if (d == 0 && p.d_bias) {
+    if (p.d_bias && part == 0) {
         float sb = 0.f;
-        constexpr int U = 8;  // eight chunks' loads in flight at a time, summed in chunk order
-        for (int ch0 = 0; ch0 < p.n_chunks; ch0 += U) {
-            float ab[U];
-#pragma unroll
-            for (int u = 0; u < U; ++u) ab[u] = p.part_b[min(ch0 + u, p.n_chunks - 1) * cstride + prow(h, sl)];
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-                if (ch0 + u < p.n_chunks) sb += ab[u];
+        for (int ch0 = 0; ch0 < p.n_chunks; ch0 += 64) {  // a chunk per lane, added in chunk order
+            const int n = min(64, p.n_chunks - ch0);
+            const float v = lane < n ? p.part_b[(ch0 + lane) * cstride + row] : 0.f;
+            for (int u = 0; u < n; ++u) sb += __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), u));
         }
-        p.d_bias[(((int64_t)h * p.num_seqs + s) * p.n_sets) * K + sl] = sb;
+        if (lane == 0) p.d_bias[row] = sb;
     }
     if (pos < 0 || pos >= len) return;
-    // only the owner of the row goes on: the first copy of the position in this set, and no
-    // earlier head of the group holding it
-    if (sl > 0 && set[sl - 1] == pos) return;
-    for (int hh = kvh * rep; hh < h; ++hh)
-        if (find_slot(p.lmk + (((int64_t)hh * p.num_seqs + s) * p.n_sets) * K, K, pos) >= 0) return;
-    const int64_t half = (int64_t)p.n_heads * p.num_seqs * K * D;
-    const int64_t so = prow(h, sl) * D + d;
-    float sk = p.lmk_stage[so], sv = p.lmk_stage[half + so];
-    for (int hh = h; hh < (kvh + 1) * rep; ++hh) {
-        const int32_t* hset = p.lmk + (((int64_t)hh * p.num_seqs + s) * p.n_sets) * K;
-        // a set may repeat a position (each copy counts, as in the forward): its copies
-        // are adjacent in the ascending set
-        for (int slot = hh == h ? sl : find_slot(hset, K, pos); slot >= 0 && slot < K && hset[slot] == pos; ++slot) {
-            const int64_t pr0 = prow(hh, slot);
-            // chunk partials in chunk order; eight chunks' loads in flight at a time
-            constexpr int U = 8;
-            for (int ch0 = 0; ch0 < p.n_chunks; ch0 += U) {
-                float ak[U], av[U];
+    if (part > 0) {  // the band sums enter once
+        sk = (vec)(0.f);
+        sv = (vec)(0.f);
+    }
+    const int cq = ceil_div(p.n_chunks, WPR);
+    const int c0 = part * cq, c1 = min(p.n_chunks, c0 + cq);
+    const float* pk = p.part_k + lane * CPL;
+    const float* pv = p.part_v + lane * CPL;
+    // partials of N slots (rows of the partials, -1: none), U chunks of each in flight
+    auto add_slots = [&](auto n_tag, auto u_tag, const int64_t* rows) {
+        constexpr int N = decltype(n_tag)::value, U = decltype(u_tag)::value;
+        vec hk[N], hv[N];
+#pragma unroll
+        for (int n = 0; n < N; ++n) hk[n] = hv[n] = (vec)(0.f);
+        for (int ch0 = c0; ch0 < c1; ch0 += U) {
+            vec ak[N][U], av[N][U];
+#pragma unroll
+            for (int n = 0; n < N; ++n)
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
-                    const int ch = min(ch0 + u, p.n_chunks - 1);
-                    const int64_t pr = ch * cstride + pr0;
-                    ak[u] = p.part_k[pr * D + d];
-                    av[u] = p.part_v[pr * D + d];
+                    ak[n][u] = av[n][u] = (vec)(0.f);
+                    if (rows[n] >= 0) {
+                        const int64_t o = (min(ch0 + u, c1 - 1) * cstride + rows[n]) * D;
+                        ak[n][u] = *(const vec*)(pk + o);
+                        av[n][u] = *(const vec*)(pv + o);
+                    }
                 }
 #pragma unroll
+            for (int n = 0; n < N; ++n)
+#pragma unroll
                 for (int u = 0; u < U; ++u)
-                    if (ch0 + u < p.n_chunks) {
-                        sk += ak[u];
-                        sv += av[u];
+                    if (ch0 + u < c1) {
+                        hk[n] += ak[n][u];
+                        hv[n] += av[n][u];
                     }
+        }
+#pragma unroll
+        for (int n = 0; n < N; ++n) {
+            sk += hk[n];
+            sv += hv[n];
+        }
+    };
+    typedef std::integral_constant<int, 1> one;
+    typedef std::integral_constant<int, HB> batch;
+    auto prow = [&](int hh, int slot) { return ((int64_t)hh * p.num_seqs + s) * K + slot; };
+    // a set may repeat a position: each copy counts, as in the forward, and its copies are
+    // adjacent in the ascending set
+    auto add_copies = [&](int hh, int slot0, int n) {
+        for (int slot = slot0; slot < slot0 + n; ++slot) {
+            const int64_t r = prow(hh, slot);
+            add_slots(one{}, std::integral_constant<int, 8>{}, &r);
+        }
+    };
+    // only the owner of the row goes on: no earlier head of the group holds the position, and
+    // this is its first copy in its own set (every wave of a row decides alike)
+    if (!wide) {
+        for (int hb = kvh * rep; hb < hend; hb += HB) {
+            if (hb > kvh * rep) load_sets(hb);
+            int first[HB], n[HB], nmax = 0;
+            int64_t rows[HB];
+#pragma unroll
+            for (int u = 0; u < HB; ++u) {
+                const uint64_t m0 = __ballot(lane < K && v0[u] == pos), m1 = __ballot(64 + lane < K && v1[u] == pos);
+                const bool any = hb + u < hend && (m0 | m1) != 0;
+                first[u] = m0 ? __builtin_ctzll(m0) : m1 ? 64 + __builtin_ctzll(m1) : 0;
+                n[u] = any ? __popcll(m0) + __popcll(m1) : 0;
+                if (any && (hb + u < h || (hb + u == h && first[u] != sl))) return;
+                rows[u] = any ? prow(hb + u, first[u]) : -1;
+                nmax = max(nmax, n[u]);
+            }
+            if (rep > 1 && nmax == 1) {
+                add_slots(batch{}, std::integral_constant<int, 4>{}, rows);
+            } else {
+#pragma unroll
+                for (int u = 0; u < HB; ++u) add_copies(hb + u, first[u], n[u]);
             }
         }
+    } else {
+        const int32_t* set = set_of(h);
+        if (sl > 0 && set[sl - 1] == pos) return;
+        for (int hh = kvh * rep; hh < h; ++hh)
+            if (find_slot(set_of(hh), K, pos) >= 0) return;
+        for (int hh = h; hh < hend; ++hh) {
+            const int32_t* hset = set_of(hh);
+            const int first = hh == h ? sl : find_slot(hset, K, pos);
+            int n = 0;
+            while (first >= 0 && first + n < K && hset[first + n] == pos) ++n;
+            add_copies(hh, first, n);
+        }
     }
-    const int64_t o = (int64_t)(st + pos) * p.n_kv_heads * D + (int64_t)kvh * D + d;
-    ((T*)p.dk)[o] = from_float<T>(sk);
-    ((T*)p.dv)[o] = from_float<T>(sv);
+    if constexpr (WPR > 1) {
+        red[(2 * wave) * 64 + lane] = sk;
+        red[(2 * wave + 1) * 64 + lane] = sv;
+        __syncthreads();
+        if (wave > 0) return;
+#pragma unroll
+        for (int w = 1; w < WPR; ++w) {
+            sk += red[(2 * w) * 64 + lane];
+            sv += red[(2 * w + 1) * 64 + lane];
+        }
+    }
+    const int64_t o = (int64_t)(st + pos) * p.n_kv_heads * D + (int64_t)kvh * D + lane * CPL;
+#pragma unroll
+    for (int c = 0; c < CPL; ++c) {
+        ((T*)p.dk)[o + c] = from_float<T>(sk[c]);
+        ((T*)p.dv)[o + c] = from_float<T>(sv[c]);
+    }
 }
 
 // training variant: d w~ per token, the per-head sums added in head order
@@ -1248,13 +1389,17 @@ hipError_t train_dw_launch(const AttnParams& p, hipStream_t stream) {
 
 // ---------------------------------------------------------------- launch
 // blocks of the landmark backward per (head, sequence, slot group): at most kRowChunk rows
-// each, and more (down to one 64-row tile each) until the launch has about sixteen waves
-// per CU, since a block's rows are one dependent chain of staged tiles
+// each, and more (down to one 64-row tile each) while every block is resident at once, since a
+// block's rows are one dependent chain of staged tiles.  Resident waves per CU: 16 of the
+// eight-wave blocks, else 12 (three per SIMD; 8 for float32 head_dim 128).  Filling past that
+// runs a second, nearly empty round of blocks and writes more partials for bwd_lmk_sum to read.
 static int lmk_chunks(const AttnParams& p) {
-    const int nw = p.dtype != DSALT_DTYPE_F32 && p.head_dim == 64 && p.k_lmk > 64 ? 8 : 4;  // as lmk_waves
+    const bool half = p.dtype != DSALT_DTYPE_F32;
+    const int nw = half && p.head_dim == 64 && p.k_lmk > 64 ? 8 : 4;  // as lmk_waves
+    const int cu_waves = nw == 8 ? 16 : (!half && p.head_dim == 128) ? 8 : 12;
     const int ngrp = ceil_div(p.k_lmk, 16 * nw);
     const int sets = max(1, p.n_heads * p.num_seqs * ngrp);
-    const int fill = ceil_div(4096 / nw, sets);
+    const int fill = 256 * cu_waves / nw / sets;
     const int rows = (p.variant & DSALT_VARIANT_LMK_SHORT) ? kRowChunk / 2 : kRowChunk;
     return max(ceil_div(p.max_seqlen, rows), min(fill, ceil_div(p.max_seqlen, 64)));
 }
@@ -1294,7 +1439,24 @@ static hipError_t bwd_run(const AttnParams& p, bool plan_given, hipStream_t stre
         if (p.w_cont) DSALT_LAUNCH("bwd_dq", (bwd_dq_kernel<T, D, BN, true>), dim3(total), dim3(256), 0, stream, p);
         else DSALT_LAUNCH("bwd_dq", (bwd_dq_kernel<T, D, BN, false>), dim3(total), dim3(256), 0, stream, p);
     }
-    if (p.n_kv_heads != p.n_heads) {
+    // grouped heads, 16-bit head_dim 64, two or four to a key/value head: side by side (the whole
+    // backward, 4/1 heads x 1024: 54.6 -> 34.7 us, 16/4 heads x 8192: 147.4 -> 132.0, 16/4 x 32768:
+    // 399.7 -> 393.0, 16/8 x 32768: 397.9 -> 382.9).  Four heads of the training variant, whose edge
+    // terms keep every wave busier, gain until the blocks fill the chip several times over (1024
+    // blocks 318.5 -> 299.4 us, 2048 blocks 519.4 -> 531.7): from 2048 blocks on they stay in order.
+    const int rep = p.n_heads / p.n_kv_heads;
+    constexpr bool kSide = sizeof(T) == 2 && D == 64;
+    if (kSide && (rep == 2 || (rep == 4 && !(p.w_cont && total_kv >= 2048)))) {
+        if constexpr (kSide) {
+            if (rep == 2) {
+                if (p.w_cont) DSALT_LAUNCH("bwd_dkdv", (bwd_dkdv_kernel<T, D, true, false, 2>), dim3(total_kv), dim3(512), 0, stream, p);
+                else DSALT_LAUNCH("bwd_dkdv", (bwd_dkdv_kernel<T, D, false, false, 2>), dim3(total_kv), dim3(512), 0, stream, p);
+            } else {
+                if (p.w_cont) DSALT_LAUNCH("bwd_dkdv", (bwd_dkdv_kernel<T, D, true, false, 4>), dim3(total_kv), dim3(1024), 0, stream, p);
+                else DSALT_LAUNCH("bwd_dkdv", (bwd_dkdv_kernel<T, D, false, false, 4>), dim3(total_kv), dim3(1024), 0, stream, p);
+            }
+        }
+    } else if (p.n_kv_heads != p.n_heads) {
         if (p.w_cont) DSALT_LAUNCH("bwd_dkdv", (bwd_dkdv_kernel<T, D, true, true>), dim3(total_kv), dim3(256), 0, stream, p);
         else DSALT_LAUNCH("bwd_dkdv", (bwd_dkdv_kernel<T, D, false, true>), dim3(total_kv), dim3(256), 0, stream, p);
     } else {
@@ -1311,9 +1473,10 @@ static hipError_t bwd_run(const AttnParams& p, bool plan_given, hipStream_t stre
             if (lk) DSALT_LAUNCH("bwd_lmk", (bwd_lmk_kernel<T, D, 4, true>), grid, dim3(256), 0, stream, p);
             else DSALT_LAUNCH("bwd_lmk", (bwd_lmk_kernel<T, D, 4>), grid, dim3(256), 0, stream, p);
         }
-        const int64_t n = (int64_t)p.n_heads * p.num_seqs * p.k_lmk * D;
-        DSALT_LAUNCH("bwd_lmk_sum", (bwd_lmk_sum_kernel<T, D>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0,
-                     stream, p);
+        const int64_t rows = (int64_t)p.n_heads * p.num_seqs * p.k_lmk;
+        const int64_t owners = rows / rep;  // about this many rows have sums to add
+        if (p.n_chunks >= kSumSplit && owners < kSumFill) DSALT_LAUNCH("bwd_lmk_sum", (bwd_lmk_sum_kernel<T, D, 4>), dim3((unsigned)rows), dim3(256), 0, stream, p);
+        else DSALT_LAUNCH("bwd_lmk_sum", (bwd_lmk_sum_kernel<T, D, 1>), dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, stream, p);
     }
     return hipGetLastError();
 }

@@ -75,3 +75,48 @@ def test_forward_tiling_by_size(lens, H, G, D, dt, block):
     heads = sorted({0, H // 2 + 1, H - 1})
     ref = _dense(q, k, v, w, cu, idx, block, heads)
     assert (out[:, heads].float() - ref).abs().max() <= 3 * UNIT[dt] * v.float().abs().max()
+
+
+@pytest.mark.parametrize("lens,H,G,D,K,dt", [
+    ([1201, 77, 1, 640], 8, 2, 64, 32, torch.float16),    # four heads of a group side by side; row sums split in four
+    ([1201, 77, 1, 640], 8, 4, 64, 128, torch.bfloat16),  # two heads side by side, largest set searched by a wave
+    ([700, 65], 16, 2, 64, 129, torch.bfloat16),          # eight heads swept in order, larger sets
+    ([2100], 12, 3, 128, 100, torch.bfloat16),            # head_dim 128: swept in order
+    ([64, 63], 4, 1, 64, 1, torch.bfloat16),              # a single tile, fewer chunks than a split
+    ([3000], 128, 32, 64, 70, torch.bfloat16),            # many owner rows: one wave a row
+    ([520, 333], 4, 1, 64, 9, torch.float32),
+])
+@pytest.mark.parametrize("train", [False, True])
+def test_grouped_gradients_equal_those_of_repeated_heads(lens, H, G, D, K, dt, train):
+    """dK / dV of grouped heads against the one-head-per-key/value-head kernels on repeated k and v,
+    summed over each group.  Both form the same products per head; the repeated heads' gradients
+    are rounded to the tensor type before the sum and the grouped ones after it, so they differ by
+    at most about (heads of a group + 2) u of the largest head's gradient (float32: sums in another
+    order, 1e-5)."""
+    q, k, v, w, cu, idx = _inputs(lens, H, G, D, K, 200, dt, seed=K)
+    rep = H // G
+    for hh in range(0, H, 2):  # half of the heads share their neighbour's set, as value norms make them do
+        idx[hh] = idx[(hh + 1) % H]
+    if K > 2:  # a repeated position in the first head's sets (ascending still)
+        idx[0, :, :, 1] = idx[0, :, :, 0]
+    g = torch.Generator(device=DEV).manual_seed(1)
+    do = torch.randn(q.shape, generator=g, device=DEV).to(dt)
+    ml = max(lens)
+    if train:
+        wc = w.float() + 0.25
+        lw = torch.randn(idx.shape, generator=g, device=DEV)
+        run = lambda kk, vv: ops.train_backward(do, q, kk, vv, *ops.train_forward(q, kk, vv, wc, cu, idx, lw, max_seqlen=ml),  # noqa: E731
+                                                wc, cu, idx, lw, max_seqlen=ml)
+    else:
+        run = lambda kk, vv: ops.attention_backward(do, q, kk, vv, *ops.attention_forward(q, kk, vv, w, cu, idx, max_seqlen=ml),  # noqa: E731
+                                                    w, cu, idx, max_seqlen=ml)
+    got, ref = run(k, v), run(k.repeat_interleave(rep, 1), v.repeat_interleave(rep, 1))
+    assert torch.equal(got[0], ref[0]) and torch.equal(got[3], ref[3])  # dq, d_bias: per query head
+    unit = (rep + 2) * UNIT[dt] if dt != torch.float32 else 1e-5
+    for a, b in ((got[1], ref[1]), (got[2], ref[2])):
+        b = b.double()
+        s = b.view(b.shape[0], G, rep, D).sum(2)
+        assert (a.double() - s).abs().max() <= unit * b.abs().max()
+    again = run(k, v)
+    for a, b in zip(got, again):
+        assert torch.equal(a, b)  # one writer per element, sums in a fixed order
