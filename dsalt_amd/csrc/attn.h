@@ -96,26 +96,39 @@ __device__ __forceinline__ void edge_terms(const AttnParams& p, float wt, int d,
 
 // The soft edge of a row with continuous window wt covers at most ceil(win_edge) band
 // keys from the unclamped window start lo_u = i - floor(wt): key lo_u + k sits at
-// wt - d = frac(wt) + k.  For win_edge <= 4 the kernels read a row's edge terms from
-// a four-entry table built once per row (no transcendentals per key).
+// wt - d = frac(wt) + k.  For win_edge <= 4 the kernels read a row's edge terms from an LDS
+// table built once per row (no transcendentals per key): entry k at offset k, zeros after
+// them (the core), and kEdgeLead zeros before a wave's 16 rows (before a later row of the wave
+// lie the zeros of the one before it), so the four keys of a lane from any offset, clamped to
+// [-4, 4], read the right entries where the mask lets them count and zeros elsewhere.  Four-way
+// selects from registers instead cost 32 VALU instructions per subtile and term, more than
+// the rest of its scores, and the registers of two row groups spilled.
 constexpr int kEdgeTab = 4;
-__device__ __forceinline__ void edge_table(const AttnParams& p, float wt, float* b, float* g) {
-    const float fr = wt - floorf(wt);
-#pragma unroll
-    for (int k = 0; k < kEdgeTab; ++k) {
-        float bb, gg;
-        edge_terms(p, fr + (float)k, 0, bb, gg);
-        b[k] = bb;
-        if (g) g[k] = gg;
+constexpr int kEdgeRow = 8, kEdgeLead = 4;
+constexpr int kEdgeWave = kEdgeLead + 16 * kEdgeRow;  // floats of a wave's table
+// offset of the row of accumulator lane `lane` in the table of wave slot `slot`
+__device__ __forceinline__ int edge_row(int slot, int lane) { return slot * kEdgeWave + kEdgeLead + (lane & 15) * kEdgeRow; }
+// writes the row's entries, one per 16-lane group (every lane of the wave calls it); grad: null
+// or a second table of d bias / d wt.  Read by the same wave only.
+__device__ __forceinline__ void edge_table(const AttnParams& p, float wt, int lane, int row, float* bias, float* grad) {
+    const int g = lane >> 4;
+    float b, d;
+    edge_terms(p, wt - floorf(wt) + (float)g, 0, b, d);
+    const bool lead = (lane & 15) == 0;
+    bias[row + g] = b;
+    bias[row + 4 + g] = 0.f;
+    if (lead) bias[row - kEdgeLead + g] = 0.f;
+    if (grad) {
+        grad[row + g] = d;
+        grad[row + 4 + g] = 0.f;
+        if (lead) grad[row - kEdgeLead + g] = 0.f;
     }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
-// table entry for key offset k from lo_u (0 from kEdgeTab on: the core)
-__device__ __forceinline__ float edge_lookup(const float* t, int k) {
-    float v = 0.f;
-#pragma unroll
-    for (int e = 0; e < kEdgeTab; ++e) v = k == e ? t[e] : v;
-    return v;
-}
+// table offset of a lane's first key, k keys from lo_u
+__device__ __forceinline__ int edge_at(int row, int k) { return row + min(max(k, -kEdgeLead), kEdgeTab); }
 
 size_t plan_bytes(const AttnParams& p);
 void plan_carve(AttnParams& p, char*& ws);  // assigns plan_perm / plan_bounds / tile_wmax from a buffer

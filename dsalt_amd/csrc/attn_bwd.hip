@@ -90,6 +90,7 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 && D == 64) ? (BN == 32 ? (TR 
     __shared__ __attribute__((aligned(16))) T Vs[2][KT::ELEMS];
     __shared__ int lpos[LCAP];
     __shared__ __attribute__((aligned(16))) float lbs[LCAP];
+    __shared__ float etb[TR ? 4 * kEdgeWave : 1], etg[TR ? 4 * kEdgeWave : 1];
     // block scalars live in the second K buffer until the first chunk is staged there
     int* red = (int*)Ks[1];
 
@@ -201,9 +202,9 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 && D == 64) ? (BN == 32 ? (TR 
         cnt = lower_bound_i(lpos, nvalid, lo);
         if (TR) wt = wt_raw;
     }
-    // soft-edge bias and window gradient of keys lou .. lou+3 (training variant)
-    float etb[TR ? kEdgeTab : 1], etg[TR ? kEdgeTab : 1];
-    if (TR) edge_table(p, wt, etb, etg);
+    // soft-edge bias and window gradient of keys lou .. lou+3 (training variant, win_edge <= 4)
+    const int eo = edge_row(uw, lane);
+    if (TR && p.edge_keys <= kEdgeTab) edge_table(p, wt, lane, eo, etb, etg);
     const int lo_edge = TR ? wLmax + p.edge_keys : wLmax;  // keys from here on carry no edge bias
     float dwacc = 0.f;
     // per-row data of the key-parallel passes, head-major: a head's rows are contiguous
@@ -349,12 +350,12 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 && D == 64) ? (BN == 32 ? (TR 
                     for (int r = 0; r < 4; ++r) ci[r] = (unsigned)(x0 + r) <= wd ? 0.f : NEG;
                     if (TR && a < lo_edge) {
                         if (p.edge_keys <= kEdgeTab) {
-                            const int k0 = a + lane_off - lou;
+                            // (a masked key's dS is 0, so its gradient entry counts for nothing)
+                            const int at = edge_at(eo, a + lane_off - lou);
 #pragma unroll
                             for (int r = 0; r < 4; ++r) {
-                                const bool out = r < tl || r > th;
-                                ci[r] = out ? NEG : edge_lookup(etb, k0 + r);
-                                eg[r] = out ? 0.f : edge_lookup(etg, k0 + r);
+                                ci[r] = (unsigned)(x0 + r) <= wd ? etb[at + r] : NEG;
+                                eg[r] = etg[at + r];
                             }
                         } else {
 #pragma unroll

@@ -84,7 +84,7 @@ struct RowGroup {
     bool valid;
     float wt;  // continuous window of the row (training variant)
     int lou;   // unclamped window start i - floor(wt) (training variant)
-    float eb[kEdgeTab];  // soft-edge bias of keys lou .. lou+3 (training variant, win_edge <= 4)
+    int eo;    // the row's entries in the soft-edge table (training variant, win_edge <= 4)
     int wlo, wLmax, whi, wHmin, wcmax, wcmin;
     // several landmark sets per block (block-causal, block_size not a multiple of 64): the
     // row's set starts at slot ls of the staged sets, its visible slots are ls .. ls+cnt-1;
@@ -140,7 +140,6 @@ __device__ __forceinline__ void plan_window(const AttnParams& p, int st, RowGrou
         rg.wt = wt;
         rg.lou = rg.i - (wi - 1);
     }
-    if (p.w_cont) edge_table(p, rg.wt, rg.eb, nullptr);
 }
 
 // The group's visible landmark counts (the set's positions in LDS).
@@ -170,13 +169,15 @@ __device__ __forceinline__ void plan_counts_sets(const int* lpos, const int* nvs
 
 // Soft-edge bias of the lane's four keys a + lane_off + r of a band subtile (training
 // variant), masked keys (r < tl, and r past the diagonal when `upper`) left at -inf.
-__device__ __forceinline__ void band_edge(const AttnParams& p, const RowGroup& R, int a, int lane_off, int tl,
-                                          bool upper, floatx4& ci) {
+__device__ __forceinline__ void band_edge(const AttnParams& p, const RowGroup& R, const float* etab, int a, int lane_off,
+                                          int tl, bool upper, floatx4& ci) {
     const int th = R.hi - a - lane_off;
     if (p.edge_keys <= kEdgeTab) {
-        const int k0 = a + lane_off - R.lou;  // key offset from the unclamped window start, r = 0
+        const float* e = etab + edge_at(R.eo, a + lane_off - R.lou);
+        // [tl, th] as one unsigned compare of r - tl (a row past the end has tl > th and fails it)
+        const unsigned wd = upper ? (unsigned)R.hi - (unsigned)R.lo : 0x7fffffffu;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) ci[r] = (r < tl || (upper && r > th)) ? -INFINITY : edge_lookup(R.eb, k0 + r);
+        for (int r = 0; r < 4; ++r) ci[r] = (unsigned)(r - tl) <= wd ? e[r] : -INFINITY;
     } else {
 #pragma unroll
         for (int r = 0; r < 4; ++r) ci[r] = (r < tl || (upper && r > th)) ? -INFINITY : edge_bias(p, R.wt, th - r);
@@ -221,8 +222,15 @@ __global__ __launch_bounds__(64 * NW, ((sizeof(T) == 2 && D == 64 && RG == 2 && 
     typedef Tile<T, D, BN, NT, (BN == 64 ? 8 : Pad<T, D>::R)> KT;
     __shared__ __attribute__((aligned(16))) T Ks[2][KT::ELEMS];
     __shared__ __attribute__((aligned(16))) T Vs[2][KT::ELEMS];
-    __shared__ int lpos[LCAP];
-    __shared__ __attribute__((aligned(16))) float lbs[LCAP];
+    __shared__ __attribute__((aligned(16))) int lbuf[2 * LCAP];
+    int* const lpos = lbuf;
+    float* const lbs = (float*)(lbuf + LCAP);
+    // soft-edge table: for one row group over the landmark slots, which the band no longer reads
+    // (the block stays at its LDS size), for two beside them
+    constexpr int kEdgeFloats = RG * NW * kEdgeWave;
+    __shared__ float ebuf[TR && RG > 1 ? kEdgeFloats : 1];
+    static_assert(!TR || RG > 1 || kEdgeFloats <= 2 * LCAP, "the soft-edge table does not fit the landmark slots");
+    float* const etab = RG > 1 ? ebuf : (float*)lbuf;
     static_assert(KT::ELEMS * sizeof(T) >= sizeof(int) * (16 + kMaxTileSets), "block scalars fit a K buffer");
     // block scalars live in the second K buffer until the first chunk is staged there
     // (keeps the block at 40 KB of LDS: four blocks per CU)
@@ -527,7 +535,7 @@ __global__ __launch_bounds__(64 * NW, ((sizeof(T) == 2 && D == 64 && RG == 2 && 
 #pragma unroll
                     for (int r = 0; r < 4; ++r) ci[r] = r < tl ? NEG : 0.f;
                     if (TR && a < R.wLmax + p.edge_keys)  // the soft edge reaches this subtile
-                        band_edge(p, R, a, lane_off, tl, false, ci);
+                        band_edge(p, R, etab, a, lane_off, tl, false, ci);
                     KOp<T, D> ko;
                     ko.load(kl, KT::RS, stt * 16, lane);
                     S[u][stt] = ko.dot(qr[u], ci);
@@ -544,7 +552,7 @@ __global__ __launch_bounds__(64 * NW, ((sizeof(T) == 2 && D == 64 && RG == 2 && 
                     floatx4 ci;
 #pragma unroll
                     for (int r = 0; r < 4; ++r) ci[r] = (unsigned)(x0 + r) <= wd ? 0.f : NEG;
-                    if (TR && a < R.wLmax + p.edge_keys) band_edge(p, R, a, lane_off, tl, true, ci);
+                    if (TR && a < R.wLmax + p.edge_keys) band_edge(p, R, etab, a, lane_off, tl, true, ci);
                     KOp<T, D> ko;
                     ko.load(kl, KT::RS, stt * 16, lane);
                     S[u][stt] = ko.dot(qr[u], ci);
@@ -647,6 +655,13 @@ __global__ __launch_bounds__(64 * NW, ((sizeof(T) == 2 && D == 64 && RG == 2 && 
         __syncthreads();
     };
     for (int n = 0; n < nlmk; ++n) process(n, std::false_type{});
+    if (TR && p.edge_keys <= kEdgeTab) {
+#pragma unroll
+        for (int u = 0; u < RG; ++u) {
+            rg[u].eo = edge_row(u * NW + uw, lane);
+            edge_table(p, rg[u].wt, lane, rg[u].eo, etab, nullptr);
+        }
+    }
     for (int n = nlmk; n < nchunks; ++n) process(n, std::true_type{});
 
     // output rows whole, staged in the idle K/V buffers (waves 0-1 in Ks, 2-3 in Vs; the
@@ -675,7 +690,7 @@ __global__ __launch_bounds__(64 * NW, ((sizeof(T) == 2 && D == 64 && RG == 2 && 
 // stay within one landmark set, block_size a multiple of 128); for 16-bit head_dim 128, two
 // row groups per wave (FWD_RG2, same condition) or 64-key chunks instead of 32 (FWD_BN64;
 // ignored with FWD_RG2);
-// fp32 takes its single compiled tiling.  With no forward bit set the operator picks by the work
+// fp32 takes its single compiled tiling.  With no forward bit set the call picks by its work
 // in 64-row tiles, tokens x heads / 64 (one call, plan included, against the 64-row tiling of
 // 64-key, at head_dim 128 32-key, chunks; windows up to 64 .. 512, 16 .. 256 landmarks):
 //   head_dim 64: FWD_RG2 | FWD_BN32 from kRg2Tiles on.  The 128-row blocks read each K and V^T
@@ -685,7 +700,8 @@ __global__ __launch_bounds__(64 * NW, ((sizeof(T) == 2 && D == 64 && RG == 2 && 
 //   head_dim 128: FWD_8W from kW8Tiles on, where staging the key chunks bounds the kernel: 32768
 //     tiles 0.945-0.997x (16 heads x 131072, 256 landmarks: 1130 -> 1077 us); 8192 tiles
 //     0.93-1.12x and 2048 0.96-1.07x (slower for windows below 512), so these keep four waves.
-// The training variant keeps its 64-row tiling (with RG2 its edge terms spill: 189 -> 335 us).
+// The training variant takes the same line (head_dim 64: 1536 tiles 0.91-0.98x, 4096 0.85-0.91x,
+// 8192 182.2 -> 154.9 us) and has no eight-wave tiling.
 // Sets of more than kSetSlots landmarks, and
 // block-causal sets of a block_size that is not a multiple of 64, take the default tiling's
 // wide instantiation (variant bits ignored).
@@ -695,10 +711,10 @@ constexpr int64_t kRg2Tiles = 1536, kW8Tiles = 16384;
 template <typename T, int D, bool TR>
 static int fwd_variant(const AttnParams& p) {
     constexpr int kFwdBits = DSALT_VARIANT_FWD_BN32 | DSALT_VARIANT_FWD_RG2 | DSALT_VARIANT_FWD_BN64 | DSALT_VARIANT_FWD_8W;
-    if (TR || sizeof(T) != 2 || (p.variant & kFwdBits) || p.block_size % 128) return p.variant;
+    if (sizeof(T) != 2 || (p.variant & kFwdBits) || p.block_size % 128) return p.variant;
     const int64_t tiles = (int64_t)p.total_len * p.n_heads / 64;
     if (D == 64) return tiles >= kRg2Tiles ? p.variant | DSALT_VARIANT_FWD_RG2 | DSALT_VARIANT_FWD_BN32 : p.variant;
-    return tiles >= kW8Tiles ? p.variant | DSALT_VARIANT_FWD_8W : p.variant;
+    return !TR && tiles >= kW8Tiles ? p.variant | DSALT_VARIANT_FWD_8W : p.variant;
 }
 
 template <typename T, int D, bool TR>

@@ -334,7 +334,7 @@ int    dsalt_sort_landmarks(const dsalt_sort_args* a, dsalt_stream_t stream);
 
 /* Tile variants of the attention kernels (dsalt_fwd_args.variant, dsalt_bwd_args.variant).
  * Bits are independent; a bit a shape cannot use is ignored.  Without forward bits the
- * operator's forward picks its tiling by the call's size (attn_fwd.hip::fwd_variant). */
+ * forward picks its tiling by the call's size (attn_fwd.hip::fwd_variant). */
 #define DSALT_VARIANT_DEFAULT    0
 #define DSALT_VARIANT_FWD_BN32   1  /* forward: 32-key chunks (16-bit types, head_dim 64)        */
 #define DSALT_VARIANT_FWD_RG2    2  /* forward: two 16-row groups per wave (16-bit types)       */
