@@ -324,12 +324,12 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 && D == 64) ? (BN == 32 ? (TR 
 #pragma unroll
         for (int stt = 0; stt < NST; ++stt) {
             const int a = base + stt * 16;
-            act[stt] = band ? (TR ? (a <= whi && a + 15 >= wlo) : cact) : (a < wcmax);
+            act[stt] = band ? cact : (a < wcmax);
             if (!act[stt]) {
                 // an inactive band chunk of the inference variant adds nothing (both subtiles
                 // share its activity, so its dS is never read); a skipped subtile beside an
                 // active one adds zeros
-                if (!band || TR) dS[stt] = floatx4{0.f, 0.f, 0.f, 0.f};
+                if (!band) dS[stt] = floatx4{0.f, 0.f, 0.f, 0.f};
                 continue;
             }
             floatx4 ci;
