@@ -111,6 +111,11 @@ class SiluMulArgs(ctypes.Structure):
                 ("up", _vp), ("up_stride", _i64), ("out", _vp), ("out_stride", _i64)]
 
 
+class SelectorsArgs(ctypes.Structure):
+    _fields_ = [("total_len", _i32), ("n_heads", _i32), ("dtype", _i32), ("gate", _vp), ("gate_stride", _i64),
+                ("alpha_w", _vp), ("n_min", _f32), ("n_span", _f32), ("w", _vp), ("alpha", _vp)]
+
+
 class SortArgs(ctypes.Structure):
     _fields_ = [("n_sets", _i64), ("k", _i32), ("idx_bytes", _i32), ("idx", _vp), ("sorted", _vp), ("perm", _vp),
                 ("bias", _vp), ("bias_sorted", _vp), ("bias_bytes", _i32)]
@@ -148,6 +153,7 @@ SIGNATURES = {
     "dsalt_train_bwd": ([ctypes.POINTER(TrainBwdArgs), _vp], ctypes.c_int),
     "dsalt_rope_qk": ([ctypes.POINTER(RopeArgs), _vp], ctypes.c_int),
     "dsalt_silu_mul": ([ctypes.POINTER(SiluMulArgs), _vp], ctypes.c_int),
+    "dsalt_layer_selectors": ([ctypes.POINTER(SelectorsArgs), _vp], ctypes.c_int),
     "dsalt_sort_landmarks": ([ctypes.POINTER(SortArgs), _vp], ctypes.c_int),
     "dsalt_export_probs": ([ctypes.POINTER(ProbsArgs), _vp], ctypes.c_int),
     "dsalt_cross_entropy_rows": ([ctypes.POINTER(CeArgs), _vp], ctypes.c_int),

@@ -29,6 +29,8 @@ SOURCES = {
     "ffn.hip": ["-ffp-contract=off"],
     "probs.hip": [],
     "sets.hip": [],
+    # one rounding per operation, as the torch expression
+    "layer.hip": ["-ffp-contract=off"],
     "ce.hip": [],
     "capi.hip": [],
     "timing.hip": [],

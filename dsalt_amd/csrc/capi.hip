@@ -10,6 +10,7 @@
 #include "attn.h"
 #include "ce.h"
 #include "ffn.h"
+#include "layer.h"
 #include "probs.h"
 #include "rope.h"
 #include "select.h"
@@ -698,6 +699,28 @@ int dsalt_sort_landmarks(const dsalt_sort_args* a, dsalt_stream_t stream) {
     p.bias_out = a->bias_sorted;
     p.bias_bytes = a->bias ? a->bias_bytes : 0;
     return hip_status(dsalt::sort_sets_launch(p, (hipStream_t)stream), "dsalt_sort_landmarks");
+}
+
+int dsalt_layer_selectors(const dsalt_selectors_args* a, dsalt_stream_t stream) {
+    if (!a) return fail(DSALT_ERR_INVALID, "null argument struct");
+    if (a->total_len < 0 || a->n_heads < 0 || (int64_t)a->total_len + a->n_heads > 0x7fffff00)
+        return fail(DSALT_ERR_INVALID, "total_len >= 0 and n_heads >= 0 required (got %d, %d)", a->total_len, a->n_heads);
+    if (a->dtype < 0 || a->dtype > 2) return fail(DSALT_ERR_INVALID, "unknown dtype %d", a->dtype);
+    if (a->total_len > 0 && (!a->gate || !a->w || a->gate_stride < 1))
+        return fail(DSALT_ERR_INVALID, "gate (positive stride) and w are required");
+    if (a->n_heads > 0 && (!a->alpha_w || !a->alpha)) return fail(DSALT_ERR_INVALID, "alpha_w and alpha are required");
+    dsalt::SelectorsParams p;
+    p.total_len = a->total_len;
+    p.n_heads = a->n_heads;
+    p.dtype = a->dtype;
+    p.gate = a->gate;
+    p.gate_st = a->gate_stride;
+    p.alpha_w = a->alpha_w;
+    p.n_min = a->n_min;
+    p.n_span = a->n_span;
+    p.w = a->w;
+    p.alpha = a->alpha;
+    return hip_status(dsalt::selectors_launch(p, (hipStream_t)stream), "dsalt_layer_selectors");
 }
 
 int dsalt_gather_landmarks(const dsalt_gather_args* a, dsalt_stream_t stream) {

@@ -41,7 +41,7 @@ from .. import ops
 from ..kernels.dsalt_attn import dsalt_attention, pad_head_dim, padded_head_dim
 from ..kernels.dsalt_train import dsalt_train_attention
 from ..kernels.landmark_tokens_ker import hybrid_scores_per_head
-from ..kernels.selectors import _compute_landmark_indices
+from ..kernels.selectors import _SCOPES, _compute_landmark_indices
 from ..kernels.window_utils import apply_rotary_emb, build_rope_cache
 
 
@@ -172,6 +172,19 @@ class DSALTAttention(nn.Module):
             self._rope32 = (key, c.float(), s.float())
         return self._rope32[1], self._rope32[2]
 
+    def _selectors(self, x):
+        """(integer windows [T] int32, alpha [H] float32) of the inference branch: one kernel after
+        the gate's product, or the torch expressions where a subclass redefines them or the tensors'
+        types differ (autocast)."""
+        cls = type(self)
+        if cls._window_sizes is DSALTAttention._window_sizes and cls._alpha is DSALTAttention._alpha \
+                and cls._window_continuous is DSALTAttention._window_continuous and x.is_cuda:
+            gate = self.win_gate(x)
+            if gate.dtype == self.alpha_w.dtype and gate.dim() == 2 and gate.shape[1] == 1 \
+                    and gate.dtype in (torch.float32, torch.bfloat16, torch.float16):
+                return ops.layer_selectors(gate.detach().view(-1), self.alpha_w.detach(), self.n_min, self.n_max)
+        return self._window_sizes(x, floor=True).to(torch.int32), self._alpha().float()
+
     @torch.no_grad()
     def _packed_inference(self, x, cu_seqlens, total_len, device, rope_cs=None, cu_list=None):
         H, G, D = self.n_heads, self.n_kv_heads, self.head_dim
@@ -187,20 +200,21 @@ class DSALTAttention(nn.Module):
         else:  # rows already gathered per token: token t reads row t
             cu1 = torch.tensor([0, total_len], dtype=torch.int32, device=device)
             ops.rope_qk_(q, k, cu1, rope_cs[0].float(), rope_cs[1].float(), max_seqlen=total_len)
-        w = self._window_sizes(x, floor=True)
-        lmk, _, _ = _compute_landmark_indices(x, self.v_proj.weight, self._alpha().float(), w, cu_seqlens, self.k_lmk,
-                                              self.n_min, total_len, cu_list, head_dim=D, select_mode=self.select_mode,
-                                              block_size=self.block_size, stats_scope=self.stats_scope)
-        idx = lmk.to(torch.int32) if lmk.dim() == 4 else lmk.to(torch.int32).unsqueeze(2)
+        w32, alpha = self._selectors(x)
         mode = ops.SELECT_BLOCK if self.select_mode == "block" else ops.SELECT_GLOBAL
-        w32 = w.to(torch.int32)
+        # landmarks on x W_V^T without the bias, whatever the projection's; the selection's first
+        # launch also writes the attention's row plan
+        plan = ops.plan_buffer(total_len, cu_seqlens.shape[0] - 1, maxlen, x.device)
+        idx = ops.select_landmarks(x, (x @ self.v_proj.weight.T).view(total_len, G, D), alpha, w32, cu_seqlens,
+                                   self.k_lmk, max_seqlen=maxlen, select_mode=mode, block_size=self.block_size,
+                                   stats_scope=_SCOPES[self.stats_scope], plan=plan)
         # head_dims other than the compiled 64 / 128 run zero-padded, scaled by the true head_dim
         dp = padded_head_dim(D)
         if dp != D:
             q, k, v = (pad_head_dim(t, dp) for t in (q, k, v))
         scale = 1.0 / math.sqrt(D)
         out, lse = ops.attention_forward(q, k, v, w32, cu_seqlens, idx, None, scale=scale, max_seqlen=maxlen,
-                                         select_mode=mode, block_size=self.block_size)
+                                         select_mode=mode, block_size=self.block_size, plan=plan, plan_ready=True)
         if dp != D:
             out = out[..., :D].contiguous()
         self._last_P = self._last_P_sparse = None

@@ -15,7 +15,7 @@ from . import _lib
 from ._lib import (DTYPE_BF16, DTYPE_F16, DTYPE_F32, SELECT_BLOCK, SELECT_GLOBAL, STATS_PACKED,
                    STATS_SEQUENCE, VARIANT_DEFAULT, VARIANT_DQ_BN64, VARIANT_FWD_BN32, VARIANT_FWD_RG2,
                    VARIANT_LMK_SHORT, BwdArgs, CeArgs, FwdArgs, GatherArgs, Problem, ProbsArgs, RopeArgs, SelectArgs,
-                   SiluMulArgs, SortArgs,
+                   SelectorsArgs, SiluMulArgs, SortArgs,
                    TrainBwdArgs,
                    TrainFwdArgs)
 
@@ -33,25 +33,41 @@ def dtype_code(dt: torch.dtype) -> int:
 
 
 def _gpu(*ts: torch.Tensor) -> torch.device:
-    dev = None
+    first, idx = None, -1
     for t in ts:
         if t is None:
             continue
-        if t.device.type != "cuda":
+        if not t.is_cuda:
             raise ValueError("dsalt_amd runs on the GPU only; got a tensor on " + str(t.device))
-        if dev is None:
-            dev = t.device
-        elif t.device != dev:
+        if first is None:
+            first, idx = t, t.get_device()
+        elif t.get_device() != idx:
             raise ValueError("all tensors must be on the same device")
-    return dev
+    return first.device if first is not None else None
 
 
 def _ptr(t):
     return ctypes.c_void_p(t.data_ptr()) if t is not None else None
 
 
+# the raw stream handle without a Stream object (a few us a call), where torch offers it
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def _stream(dev: torch.device):
-    return ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+    if _raw_stream is not None and dev.index is not None:
+        return _raw_stream(dev.index)
+    return torch.cuda.current_stream(dev).cuda_stream
+
+
+def _i32(t: torch.Tensor) -> torch.Tensor:
+    """``t`` as a contiguous int32 tensor (itself when it is one)."""
+    return t if t.dtype == torch.int32 and t.is_contiguous() else t.detach().to(torch.int32).contiguous()
+
+
+def _f32(t: torch.Tensor) -> torch.Tensor:
+    """``t`` as a contiguous float32 tensor (itself when it is one)."""
+    return t if t.dtype == torch.float32 and t.is_contiguous() else t.detach().to(torch.float32).contiguous()
 
 
 def _rows3(t: torch.Tensor, name: str) -> torch.Tensor:
@@ -61,6 +77,11 @@ def _rows3(t: torch.Tensor, name: str) -> torch.Tensor:
     if t.stride(2) != 1:
         t = t.contiguous()
     return t
+
+
+def _rows_ptr(t: torch.Tensor):
+    """(address, token stride, head stride) of a [T, H, D] tensor."""
+    return (t.data_ptr(), *t.stride()[:2])
 
 
 def _check_tokens(q, k, v, w, cu_seqlens):
@@ -144,26 +165,22 @@ def select_landmarks(h: torch.Tensor, v: torch.Tensor, alpha: torch.Tensor, w: t
         raise ValueError(f"k_lmk must be in [0, {MAX_LANDMARKS}]")
     maxlen = max_seqlen if max_seqlen is not None else _max_seqlen(cu_seqlens)
     nset = n_sets(select_mode, maxlen, block_size)
-    alpha_c = alpha.detach().to(torch.float32).contiguous()
-    w_c = w.detach().to(torch.int32).contiguous()
-    cu_c = cu_seqlens.detach().to(torch.int32).contiguous()
+    alpha_c = _f32(alpha)
+    w_c = _i32(w)
+    cu_c = _i32(cu_seqlens)
     idx = torch.empty((H, S, nset, k_lmk), dtype=torch.int32, device=dev)
     zx = zv = sc = None
     if want_scores:
         zx = torch.empty(T, dtype=torch.float32, device=dev)
         zv = torch.empty((T, G), dtype=torch.float32, device=dev)
         sc = torch.empty((T, H), dtype=torch.float32, device=dev)
-    a = SelectArgs()
-    a.p = _problem(T, S, maxlen, H, G, D, k_lmk, select_mode, block_size, dt)
-    a.hidden, a.stats_scope = hidden, stats_scope
-    a.h, a.h_stride_t = h.data_ptr(), h.stride(0)
-    a.v, a.v_stride_t, a.v_stride_h = v.data_ptr(), v.stride(0), v.stride(1)
-    a.alpha, a.w, a.cu_seqlens = alpha_c.data_ptr(), w_c.data_ptr(), cu_c.data_ptr()
-    a.lmk_idx = idx.data_ptr() if idx.numel() else None
-    a.z_x = zx.data_ptr() if zx is not None else None
-    a.z_v = zv.data_ptr() if zv is not None else None
-    a.scores = sc.data_ptr() if sc is not None else None
-    a.plan = _check_plan(plan, a) or None
+    a = SelectArgs(_problem(T, S, maxlen, H, G, D, k_lmk, select_mode, block_size, dt), hidden, stats_scope,
+                   h.data_ptr(), h.stride(0), *_rows_ptr(v), alpha_c.data_ptr(), w_c.data_ptr(), cu_c.data_ptr(),
+                   idx.data_ptr() if idx.numel() else None)
+    if want_scores:
+        a.z_x, a.z_v, a.scores = zx.data_ptr(), zv.data_ptr(), sc.data_ptr()
+    if plan is not None:
+        a.plan = _check_plan(plan, a) or None
     L = _lib.load()
     if border_cap is None:
         need = L.dsalt_select_workspace_bytes(ctypes.byref(a))
@@ -205,23 +222,17 @@ def _fwd_args(q, k, v, w, cu_seqlens, lmk_idx, lmk_bias, scale, max_seqlen, sele
     if lmk_idx.shape[2] != n_sets(select_mode, maxlen, block_size):
         raise ValueError("lmk_idx n_sets does not match select_mode / block_size / max_seqlen")
     scale = 1.0 / math.sqrt(D) if scale is None else float(scale)
-    w_c = w.detach().to(torch.int32).contiguous() if need_w else None
-    cu_c = cu_seqlens.detach().to(torch.int32).contiguous()
-    li = lmk_idx.to(torch.int32).contiguous()
-    lb = lmk_bias.detach().to(torch.float32).contiguous() if lmk_bias is not None else None
+    w_c = _i32(w) if need_w else None
+    cu_c = _i32(cu_seqlens)
+    li = _i32(lmk_idx)
+    lb = _f32(lmk_bias) if lmk_bias is not None else None
     out = torch.empty((T, H, D), dtype=q.dtype, device=dev)
     lse = torch.empty((T, H), dtype=torch.float32, device=dev)
-    a = FwdArgs()
-    a.p = _problem(T, S, maxlen, H, G, D, K, select_mode, block_size, dt)
-    a.q, a.q_stride_t, a.q_stride_h = q.data_ptr(), q.stride(0), q.stride(1)
-    a.k, a.k_stride_t, a.k_stride_h = k.data_ptr(), k.stride(0), k.stride(1)
-    a.v, a.v_stride_t, a.v_stride_h = v.data_ptr(), v.stride(0), v.stride(1)
-    a.w = w_c.data_ptr() if w_c is not None else None
-    a.cu_seqlens = cu_c.data_ptr()
-    a.lmk_idx = li.data_ptr() if li.numel() else None
-    a.lmk_bias = lb.data_ptr() if lb is not None and lb.numel() else None
-    a.out, a.o_stride_t, a.o_stride_h = out.data_ptr(), out.stride(0), out.stride(1)
-    a.lse, a.scale = lse.data_ptr(), scale
+    # (positional: one pass over the fields, where attribute stores cost most of a small call)
+    a = FwdArgs(_problem(T, S, maxlen, H, G, D, K, select_mode, block_size, dt), *_rows_ptr(q), *_rows_ptr(k),
+                *_rows_ptr(v), w_c.data_ptr() if w_c is not None else None, cu_c.data_ptr(),
+                li.data_ptr() if K and li.numel() else None, lb.data_ptr() if lb is not None and lb.numel() else None,
+                out.data_ptr(), H * D, D, lse.data_ptr(), scale)
     return a, out, lse, (q, k, v, w_c, cu_c, li, lb)
 
 
@@ -235,6 +246,12 @@ def new_plan(q: torch.Tensor, k: torch.Tensor, cu_seqlens: torch.Tensor, lmk_idx
                     dtype_code(q.dtype))
     n = _lib.load().dsalt_plan_bytes(ctypes.byref(prob))
     return torch.empty(max(n, 1), dtype=torch.uint8, device=q.device)
+
+
+def plan_buffer(T: int, S: int, max_seqlen: int, device) -> torch.Tensor:
+    """An empty row-plan buffer from the batch's shape alone (as new_plan, before any landmarks)."""
+    prob = _problem(T, S, max_seqlen, 1, 1, 64, 0, SELECT_GLOBAL, 0, DTYPE_F32)
+    return torch.empty(max(_lib.load().dsalt_plan_bytes(ctypes.byref(prob)), 1), dtype=torch.uint8, device=device)
 
 
 def _check_plan(plan, a) -> int:
@@ -283,7 +300,7 @@ def _check_out_f32(t: torch.Tensor, out: torch.Tensor):
 def _w_cont(w_cont: torch.Tensor, T: int) -> torch.Tensor:
     if w_cont.dim() != 1 or w_cont.shape[0] != T:
         raise ValueError("w_cont must be [T]")
-    return w_cont.detach().to(torch.float32).contiguous()
+    return _f32(w_cont)
 
 
 def train_forward(q, k, v, w_cont, cu_seqlens, lmk_idx, lmk_logw, *, tau_win=1.0, win_edge=4.0, scale=None,
@@ -339,29 +356,20 @@ def _bwd_args(dout, q, k, v, out, lse, w, cu_seqlens, lmk_idx, lmk_bias, scale, 
     if lmk_bias is not None and tuple(lmk_bias.shape) != tuple(lmk_idx.shape):
         raise ValueError("lmk_bias must have the shape of lmk_idx")
     scale = 1.0 / math.sqrt(D) if scale is None else float(scale)
-    w_c = w.detach().to(torch.int32).contiguous() if need_w else None
-    cu_c = cu_seqlens.detach().to(torch.int32).contiguous()
-    li = lmk_idx.to(torch.int32).contiguous()
-    lb = lmk_bias.detach().to(torch.float32).contiguous() if lmk_bias is not None else None
-    lse = lse.detach().to(torch.float32).contiguous()
+    w_c = _i32(w) if need_w else None
+    cu_c = _i32(cu_seqlens)
+    li = _i32(lmk_idx)
+    lb = _f32(lmk_bias) if lmk_bias is not None else None
+    lse = _f32(lse)
     dq = torch.empty((T, H, D), dtype=q.dtype, device=dev)
     dk = torch.empty((T, G, D), dtype=q.dtype, device=dev)
     dv = torch.empty((T, G, D), dtype=q.dtype, device=dev)
     db = torch.empty(tuple(lmk_idx.shape), dtype=torch.float32, device=dev) if want_dbias else None
-    a = BwdArgs()
-    a.p = _problem(T, S, maxlen, H, G, D, K, SELECT_GLOBAL, 0, dt)
-    a.q, a.q_stride_t, a.q_stride_h = q.data_ptr(), q.stride(0), q.stride(1)
-    a.k, a.k_stride_t, a.k_stride_h = k.data_ptr(), k.stride(0), k.stride(1)
-    a.v, a.v_stride_t, a.v_stride_h = v.data_ptr(), v.stride(0), v.stride(1)
-    a.out, a.o_stride_t, a.o_stride_h = out.data_ptr(), out.stride(0), out.stride(1)
-    a.dout, a.do_stride_t, a.do_stride_h = dout.data_ptr(), dout.stride(0), dout.stride(1)
-    a.lse, a.cu_seqlens = lse.data_ptr(), cu_c.data_ptr()
-    a.w = w_c.data_ptr() if w_c is not None else None
-    a.lmk_idx = li.data_ptr() if li.numel() else None
-    a.lmk_bias = lb.data_ptr() if lb is not None and lb.numel() else None
-    a.dq, a.dk, a.dv = dq.data_ptr(), dk.data_ptr(), dv.data_ptr()
-    a.d_bias = db.data_ptr() if db is not None and db.numel() else None
-    a.scale = scale
+    a = BwdArgs(_problem(T, S, maxlen, H, G, D, K, SELECT_GLOBAL, 0, dt), *_rows_ptr(q), *_rows_ptr(k), *_rows_ptr(v),
+                *_rows_ptr(out), *_rows_ptr(dout), lse.data_ptr(), w_c.data_ptr() if w_c is not None else None,
+                cu_c.data_ptr(), li.data_ptr() if K and li.numel() else None,
+                lb.data_ptr() if lb is not None and lb.numel() else None, dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
+                db.data_ptr() if db is not None and db.numel() else None, scale)
     return a, dq, dk, dv, db, d32, (q, k, v, out, dout, w_c, cu_c, li, lb, lse)
 
 
@@ -446,8 +454,8 @@ def gather_landmarks(k, v, cu_seqlens, lmk_idx, *, max_seqlen=None, select_mode=
     if lmk_idx.dim() != 4 or lmk_idx.shape[1] != S or lmk_idx.shape[2] != n_sets(select_mode, maxlen, block_size):
         raise ValueError(f"lmk_idx must be [H, S, n_sets, K] matching select_mode/block_size, got "
                          f"{tuple(lmk_idx.shape)}")
-    li = lmk_idx.to(torch.int32).contiguous()
-    cu_c = cu_seqlens.detach().to(torch.int32).contiguous()
+    li = _i32(lmk_idx)
+    cu_c = _i32(cu_seqlens)
     shape = tuple(lmk_idx.shape) + (D,)
     lk = torch.empty(shape, dtype=k.dtype, device=dev)
     lv = torch.empty(shape, dtype=k.dtype, device=dev)
@@ -482,7 +490,7 @@ def rope_qk_(q, k, cu_seqlens, cos, sin, *, max_seqlen=None):
             or cos.shape[1] != D:
         raise ValueError("cos/sin must be float32 [max_pos, head_dim]")
     cos, sin = cos.contiguous(), sin.contiguous()
-    cu_c = cu_seqlens.detach().to(torch.int32).contiguous()
+    cu_c = _i32(cu_seqlens)
     maxlen = max_seqlen if max_seqlen is not None else _max_seqlen(cu_seqlens)
     a = RopeArgs()
     a.total_len, a.num_seqs, a.max_seqlen = T, cu_c.shape[0] - 1, maxlen
@@ -522,11 +530,11 @@ def export_probs(q, k, w, cu_seqlens, lmk_idx, lse, lmk_bias=None, *, seq=0, row
     K = lmk_idx.shape[-1]
     if lmk_idx.dim() != 4 or lmk_idx.shape[:2] != (H, S) or lmk_idx.shape[2] != n_sets(select_mode, maxlen, block_size):
         raise ValueError(f"lmk_idx must be [H, S, n_sets, K], got {tuple(lmk_idx.shape)}")
-    w_c = w.detach().to(torch.int32).contiguous()
-    cu_c = cu_seqlens.detach().to(torch.int32).contiguous()
-    li = lmk_idx.to(torch.int32).contiguous()
-    lb = lmk_bias.detach().to(torch.float32).contiguous() if lmk_bias is not None else None
-    lse_c = lse.detach().to(torch.float32).contiguous()
+    w_c = _i32(w)
+    cu_c = _i32(cu_seqlens)
+    li = _i32(lmk_idx)
+    lb = _f32(lmk_bias) if lmk_bias is not None else None
+    lse_c = _f32(lse)
     alloc = torch.empty if rows == seq_len else torch.zeros  # the kernel writes every row of the sequence
     p_win = alloc((H, rows, w_cap), dtype=torch.float32, device=dev)
     p_lmk = alloc((H, rows, K), dtype=torch.float32, device=dev) if want_lmk and K else None
@@ -636,6 +644,25 @@ def silu_mul(gate: torch.Tensor, up: torch.Tensor, out: torch.Tensor | None = No
     L = _lib.load()
     _lib.check("dsalt_silu_mul", L.dsalt_silu_mul(ctypes.byref(a), _stream(dev)))
     return out
+
+
+def layer_selectors(gate: torch.Tensor, alpha_w: torch.Tensor, n_min, n_max):
+    """(w [T] int32, alpha [H] float32) of an attention layer: w = max(floor(n_min + sigmoid(gate)
+    (n_max - n_min)), 1) from the window-gate logits ``gate`` [T], alpha = sigmoid(alpha_w), every
+    operation rounded to the tensors' type as the torch expressions."""
+    dev = _gpu(gate, alpha_w)
+    if gate.dim() != 1 or alpha_w.dim() != 1 or gate.dtype != alpha_w.dtype:
+        raise ValueError("gate must be [T] and alpha_w [H], of one dtype")
+    if gate.shape[0] > 1 and gate.stride(0) < 1:
+        gate = gate.contiguous()
+    alpha_w = alpha_w.contiguous()
+    T, H = gate.shape[0], alpha_w.shape[0]
+    w = torch.empty(T, dtype=torch.int32, device=dev)
+    alpha = torch.empty(H, dtype=torch.float32, device=dev)
+    a = SelectorsArgs(T, H, dtype_code(gate.dtype), gate.data_ptr(), gate.stride(0), alpha_w.data_ptr(), float(n_min),
+                      float(n_max - n_min), w.data_ptr(), alpha.data_ptr())
+    _lib.check("dsalt_layer_selectors", _lib.load().dsalt_layer_selectors(ctypes.byref(a), _stream(dev)))
+    return w, alpha
 
 
 def sort_landmarks(idx: torch.Tensor, bias: torch.Tensor | None = None):

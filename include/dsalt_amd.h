@@ -314,6 +314,25 @@ typedef struct dsalt_silu_mul_args {
 
 int    dsalt_silu_mul(const dsalt_silu_mul_args* a, dsalt_stream_t stream);
 
+/* Integer windows and score weights of an attention layer (dsalt/modules/dsalt_attention.py:
+ * 228,243-244,277-284): w[t] = max(floor(n_min + sigmoid(gate[t]) * n_span), 1) with
+ * n_span = n_max - n_min, alpha[h] = sigmoid(alpha_w[h]); every operation rounded to the
+ * tensor type of gate and alpha_w (which share it). */
+typedef struct dsalt_selectors_args {
+    int32_t total_len;
+    int32_t n_heads;
+    int32_t dtype;             /* DSALT_DTYPE_*                                      */
+    const void* gate;          /* [T] with element stride gate_stride                */
+    int64_t gate_stride;
+    const void* alpha_w;       /* [H]                                                */
+    float n_min;
+    float n_span;
+    int32_t* w;                /* [T] out                                            */
+    float* alpha;              /* [H] out                                            */
+} dsalt_selectors_args;
+
+int    dsalt_layer_selectors(const dsalt_selectors_args* a, dsalt_stream_t stream);
+
 /* Landmark sets in any order put into the one dsalt_fwd / dsalt_bwd take: positions
  * ascending, empty slots (any negative value) as -1 at the end; equal positions keep their
  * order.  perm is the source slot of each output slot; bias (optional) follows the same
