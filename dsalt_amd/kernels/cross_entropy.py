@@ -37,6 +37,32 @@ def _chunk_rows(BT: int, V: int, elem: int) -> int:
     return max(1, min(BT, rows))
 
 
+# Layouts of the 16-bit products (4001 rows, hidden 2048, vocabulary 151936, us): the weight
+# gradient reduces over rows, 2302 with the hidden states as they are, 1971 with them copied
+# row-contiguous (40) and the rows in whole 64-row tiles, where an odd row count also puts the
+# logits (1862 -> 1837) and the input gradient (1883 -> 1874) on edge-tile kernels; written by the
+# first chunk's product instead of added to zeros, about 170 less.  From _TILE_ROWS rows on: 1001
+# rows 2186 -> 2062 for the three (hidden 512, vocabulary 50257: 429 -> 404), 769 rows there
+# 376 -> 394, the added rows costing more than the layout gives.
+_TILE_ROWS = 960
+
+
+def _whole_rows(BT: int, chunk: int) -> int:
+    """BT with its last chunk rounded up to whole 64-row tiles (chunks are whole already)."""
+    last = BT - (BT - 1) // chunk * chunk if BT else 0
+    return BT + (-last) % 64 if last >= _TILE_ROWS else BT
+
+
+def _logits(x, w, b, V):
+    """x w^T (+ b) [rows, V] with rows on 16-byte boundaries, as the row kernel reads them (any
+    vocabulary size)."""
+    vec = 16 // x.element_size()
+    if V % vec == 0 or w.dtype != x.dtype or torch.is_autocast_enabled():
+        return torch.nn.functional.linear(x, w, b).contiguous()
+    out = torch.empty((x.shape[0], -(-V // vec) * vec), dtype=x.dtype, device=x.device)[:, :V]
+    return torch.mm(x, w.t(), out=out) if b is None else torch.addmm(b, x, w.t(), out=out)
+
+
 def fused_linear_cross_entropy_forward(_input, weight, target, ce_weight=None, bias=None, ignore_index=-100,
                                        lse_square_scale=0.0, label_smoothing=0.0, reduction="mean", softcap=None,
                                        return_z_loss=False, accum_dtype=None, use_token_scaling=False,
@@ -58,12 +84,17 @@ def fused_linear_cross_entropy_forward(_input, weight, target, ce_weight=None, b
         sum_w = float(ce_weight[tgt[keep]].sum().item())
         w_sum = float(ce_weight.sum().item())
     need_grad = _input.requires_grad
-    grad_input = torch.zeros_like(_input) if need_grad else None
+    half = _input.element_size() == 2 and weight.dtype == _input.dtype
+    chunk = _chunk_rows(BT, V, _input.element_size())
+    # rows the last chunk's products run over (whole tiles), and the gradient buffer over them
+    BTp = _whole_rows(BT, chunk) if need_grad and half else BT
+    grad_input = torch.empty((BTp, H), dtype=_input.dtype, device=dev) if need_grad else None
     grad_weight = grad_bias = None
     if need_grad:
         wd = accum_dtype if accum_dtype is not None else weight.dtype
-        if weight.requires_grad:
-            grad_weight = torch.zeros(weight.shape, dtype=wd, device=dev)
+        if weight.requires_grad:  # in the logits' type the first chunk's product writes it whole
+            alloc = torch.empty if wd == _input.dtype and BT else torch.zeros
+            grad_weight = alloc(weight.shape, dtype=wd, device=dev)
         if bias is not None:
             grad_bias = torch.zeros(bias.shape, dtype=wd, device=dev)
     loss_1d = torch.zeros(BT, dtype=torch.float32, device=dev)
@@ -72,13 +103,17 @@ def fused_linear_cross_entropy_forward(_input, weight, target, ce_weight=None, b
     pred_1d = torch.full((BT,), -1, dtype=torch.int64, device=dev) if return_predicted_tokens else None
     x = _input.detach()
     wt = weight.detach()
-    chunk = _chunk_rows(BT, V, _input.element_size())
+    bs = bias.detach() if bias is not None else None
     for s0 in range(0, BT, chunk):
         s1 = min(BT, s0 + chunk)
+        n = s1 - s0
+        m = n if s1 < BT else BTp - s0
         xc = x[s0:s1]
-        logits = torch.nn.functional.linear(xc, wt, bias.detach() if bias is not None else None).contiguous()
+        if m > n:  # zero rows up to whole tiles
+            xc = torch.cat([xc, xc.new_zeros((m - n, H))])
+        logits = _logits(xc, wt, bs, V)
         l, z, a, p = ops.cross_entropy_rows(
-            logits, tgt[s0:s1], ce_weight=ce_weight, ignore_index=ignore_index, n_non_ignore=float(n_non_ignore),
+            logits[:n], tgt[s0:s1], ce_weight=ce_weight, ignore_index=ignore_index, n_non_ignore=float(n_non_ignore),
             sum_non_ignore_weight=sum_w, weight_sum=w_sum, lse_square_scale=lse_square_scale,
             label_smoothing=label_smoothing, softcap=softcap, reduction=reduction, want_grad=need_grad,
             token_scaling=use_token_scaling, want_z=return_z_loss, want_accuracy=return_token_accuracy,
@@ -91,14 +126,21 @@ def fused_linear_cross_entropy_forward(_input, weight, target, ce_weight=None, b
         if pred_1d is not None:
             pred_1d[s0:s1] = p
         if need_grad:  # logits now hold d loss / d logits
-            torch.mm(logits, wt, out=grad_input[s0:s1])
+            if m > n:
+                logits[n:].zero_()
+            torch.mm(logits, wt, out=grad_input[s0:s0 + m])
             if grad_weight is not None:
-                if grad_weight.dtype == logits.dtype:
-                    grad_weight.addmm_(logits.t(), xc)
+                xg = xc.t().contiguous().t() if half and m >= _TILE_ROWS else xc
+                if grad_weight.dtype != logits.dtype:
+                    grad_weight += torch.mm(logits.t(), xg).to(grad_weight.dtype)
+                elif s0 == 0:
+                    torch.mm(logits.t(), xg, out=grad_weight)
                 else:
-                    grad_weight += torch.mm(logits.t(), xc).to(grad_weight.dtype)
+                    grad_weight.addmm_(logits.t(), xg)
             if grad_bias is not None:
-                grad_bias += logits.sum(dim=0).to(grad_bias.dtype)
+                grad_bias += logits[:n].sum(dim=0).to(grad_bias.dtype)
+    if need_grad:
+        grad_input = grad_input[:BT]
     if reduction == "none":
         loss, z_loss = loss_1d, z_1d
         token_accuracy = acc_1d
