@@ -206,12 +206,31 @@ __device__ __forceinline__ void mean_std(double s1, double s2, int n, double& me
 // r0 + t + kSumParts m in increasing m), then a halving tree.
 constexpr int kSumParts = 1024;
 
+// The halving tree over the kSumParts partials a[] (LDS) by one wave, every lane of it: the four
+// levels across waves pair partials 64 apart, so lane l folds its 16 partials l + 64 k in
+// registers, and the six levels below are lane shuffles (the same additions as a tree over the
+// block, without its ten barriers).  Returns the total in lane 0.
+__device__ __forceinline__ double wave_tree(const double* a, int lane) {
+    constexpr int N = kSumParts / 64;
+    double v[N];
+#pragma unroll
+    for (int k = 0; k < N; ++k) v[k] = a[lane + 64 * k];
+#pragma unroll
+    for (int off = N / 2; off >= 1; off >>= 1)
+#pragma unroll
+        for (int k = 0; k < off; ++k) v[k] = __dadd_rn(v[k], v[k + off]);
+    double t = v[0];
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) t = __dadd_rn(t, __shfl_down(t, off, 64));
+    return t;
+}
+
 __global__ __launch_bounds__(256) void sel_sums_kernel(SelectParams p, const float* nx, const float* nv,
                                                        double* sums, double* stats) {
     // thread t owns partials t + 256 q (q = 0..3), U chain steps of each in flight; reads past
     // the range return zero, and adding +0 to these sums of non-negative norms changes no bit
     constexpr int Q = kSumParts / 256, U = 8;
-    __shared__ double a1[kSumParts], a2[kSumParts];
+    __shared__ double a1[kSumParts], a2[kSumParts], tot[2];
     const int r = blockIdx.x, sig = blockIdx.y, t = threadIdx.x;
     const float* x = sig == 0 ? nx : nv + (int64_t)(sig - 1) * p.total_len;
     int r0, r1;
@@ -245,21 +264,19 @@ __global__ __launch_bounds__(256) void sel_sums_kernel(SelectParams p, const flo
         a2[t + 256 * q] = s2[q];
     }
     __syncthreads();
-    for (int off = kSumParts / 2; off >= 1; off >>= 1) {
-        for (int i = t; i < off; i += 256) {
-            a1[i] = __dadd_rn(a1[i], a1[i + off]);
-            a2[i] = __dadd_rn(a2[i], a2[i + off]);
-        }
-        __syncthreads();
+    if (t < 128) {
+        const double total = wave_tree(t < 64 ? a1 : a2, t & 63);
+        if ((t & 63) == 0) tot[t >> 6] = total;
     }
+    __syncthreads();
     if (t == 0) {
         const int nsig = 1 + p.n_kv_heads;
         const int64_t o = ((int64_t)r * nsig + sig) * 2;
-        sums[o] = a1[0];
-        sums[o + 1] = a2[0];
+        sums[o] = tot[0];
+        sums[o + 1] = tot[1];
         if (stats) {  // global variant: statistics of this range
             double m = 0.0, sd = 1.0;
-            if (r1 > r0) mean_std(a1[0], a2[0], r1 - r0, m, sd);
+            if (r1 > r0) mean_std(tot[0], tot[1], r1 - r0, m, sd);
             stats[o] = m;
             stats[o + 1] = sd;
         }
@@ -763,11 +780,16 @@ __global__ __launch_bounds__(256) void sel_prune_list_kernel(SelectParams p, con
 constexpr int kPartMax = 2048;   // candidates per part (keys in LDS)
 constexpr int kMergeMax = 4096;  // keys per merge block
 
+// Statistics (mean, std, 1 / std) of the two signals of a set.
+struct SetStats {
+    double mean[2], sd[2], rsd[2];
+};
+
 // key of set (h, sequence s starting at st): z-scores from the norms and the range's
 // statistics (mean, std of the hidden-state and value-vector norms; the same values sel_z
 // stores)
 __device__ __forceinline__ KeyFn global_key_of(const SelectParams& p, const float* nx, const float* nv, int st, int h,
-                                               double mx, double sx, double mv, double sv) {
+                                               const SetStats& ss) {
     KeyFn key;
     key.w = p.w;
     key.total_len = p.total_len;
@@ -781,12 +803,12 @@ __device__ __forceinline__ KeyFn global_key_of(const SelectParams& p, const floa
     key.nx = nx;
     key.nv = nv;
     key.pk = nullptr;
-    key.mx = mx;
-    key.sx = sx;
-    key.mv = mv;
-    key.sv = sv;
-    key.rsx = __ddiv_rn(1.0, key.sx);
-    key.rsv = __ddiv_rn(1.0, key.sv);
+    key.mx = ss.mean[0];
+    key.sx = ss.sd[0];
+    key.mv = ss.mean[1];
+    key.sv = ss.sd[1];
+    key.rsx = ss.rsd[0];
+    key.rsv = ss.rsd[1];
     return key;
 }
 
@@ -806,10 +828,11 @@ __device__ __forceinline__ int global_range(const SelectParams& p, int s) {
 
 // Statistics of range r for the hidden-state norms (q = 0) and the norms of value head g
 // (q = 1), computed by one 1024-thread block in sel_sums' canonical order: thread t sums
-// partial t of both signals, then the halving tree, then mean_std.  The global top-k parts
-// use it when no caller asked for z or scores, so no sel_sums launch precedes them.
-__device__ void pair_stats(const SelectParams& p, const float* nx, const float* nv, int r, int g, double (&mean)[2],
-                           double (&sd)[2]) {
+// partial t of both signals, then the halving tree and mean_std by one wave per signal (its
+// dozen float64 divisions by every wave were a third of the kernel for short sequences).  The
+// global top-k parts use it when no caller asked for z or scores, so no sel_sums launch
+// precedes them.  Ends with a barrier after which `out` (LDS) is set.
+__device__ void pair_stats(const SelectParams& p, const float* nx, const float* nv, int r, int g, SetStats& out) {
     static_assert(kSelThreads == kSumParts, "one partial per thread");
     constexpr int U = 16;
     __shared__ double a1[2][kSumParts], a2[2][kSumParts];
@@ -831,13 +854,15 @@ __device__ void pair_stats(const SelectParams& p, const float* nx, const float* 
                                               __builtin_amdgcn_raw_buffer_load_b32(rs, (uint32_t)(t + kSumParts * m) * 4u, 0, 0));
         }
 #pragma unroll
-        for (int m = 0; m < U; ++m)
+        for (int m = 0; m < U; ++m) {
+            if (m * kSumParts >= n) break;  // past the range: zeros, which change no sum
 #pragma unroll
             for (int q = 0; q < 2; ++q) {
                 const double v = (double)xv[q][m];
                 s1[q] = __dadd_rn(s1[q], v);
                 s2[q] = __dadd_rn(s2[q], __dmul_rn(v, v));
             }
+        }
     }
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
@@ -845,22 +870,18 @@ __device__ void pair_stats(const SelectParams& p, const float* nx, const float* 
         a2[q][t] = s2[q];
     }
     __syncthreads();
-    for (int off = kSumParts / 2; off >= 1; off >>= 1) {
-        if (t < off) {
-#pragma unroll
-            for (int q = 0; q < 2; ++q) {
-                a1[q][t] = __dadd_rn(a1[q][t], a1[q][t + off]);
-                a2[q][t] = __dadd_rn(a2[q][t], a2[q][t + off]);
-            }
+    if (t < 128) {
+        const int q = t >> 6, lane = t & 63;
+        const double t1 = wave_tree(a1[q], lane), t2 = wave_tree(a2[q], lane);
+        if (lane == 0) {
+            double m = 0.0, sd = 1.0;
+            if (r1 > r0) mean_std(t1, t2, r1 - r0, m, sd);
+            out.mean[q] = m;
+            out.sd[q] = sd;
+            out.rsd[q] = __ddiv_rn(1.0, sd);
         }
-        __syncthreads();
     }
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {
-        mean[u] = 0.0;
-        sd[u] = 1.0;
-        if (r1 > r0) mean_std(a1[u][0], a2[u][0], r1 - r0, mean[u], sd[u]);
-    }
+    __syncthreads();
 }
 
 // Writes the kpad largest of the n keys a[0..n) (LDS) to o, in no particular order: the keys
@@ -881,39 +902,66 @@ __device__ void keep_largest(KthShared& sh, const unsigned long long* a, int n, 
     for (int i = (int)sh.ncand + tid; i < kpad; i += kSelThreads) o[i] = kk;
 }
 
-// part q of set (h, s): candidates [q*psize, (q+1)*psize); writes its kpad best keys
-// (zero keys where it has fewer)
 constexpr int kSortThreads = kSelThreads;
 
+// The set's landmark indices (ascending, -1 padded) from the n keys keys[0..n) (LDS) of its
+// candidates: the K largest -- those above the K-th largest, and it when it is a candidate's
+// key (keys of candidates are distinct; fewer than K candidates leave it 0).
+__device__ __forceinline__ void write_set(const SelectParams& p, KthShared& sh, const unsigned long long* keys, int n,
+                                          int* sel, int sidx, int tid) {
+    const int K = p.k_lmk;
+    const unsigned long long kk = n > K ? kth_desc(sh, keys, n, K - 1, tid) : 0ull;
+    if (tid == 0) sh.ncand = 0u;
+    __syncthreads();
+    for (int i = tid; i < n; i += kSortThreads) {
+        const unsigned long long kj = keys[i];
+        if (kj > kk || (kj == kk && kk != 0ull))
+            sel[atomicAdd(&sh.ncand, 1u)] = (int)(0xffffffffu - (uint32_t)(kj & 0xffffffffull));
+    }
+    __syncthreads();
+    const int nsel = (int)sh.ncand;
+    int32_t* o = p.lmk_idx + (int64_t)sidx * K;
+    rank_sort_asc<kSelThreads>(sel, nsel, o, tid);
+    for (int i = nsel + tid; i < K; i += kSortThreads) o[i] = -1;
+}
+
+// part q of set (h, s): candidates [q*psize, (q+1)*psize); writes its kpad best keys
+// (zero keys where it has fewer).  KCAP > 0: the set has one part (sequences of up to psize
+// tokens), and the block writes its at most KCAP indices itself, no merge launch after it.
+// Selection of 4 heads x 2048: part 12.7 + merge 4.4 -> 10.1 us (8/2 heads of 5 short sequences: 12.9 + 5.2 -> 10.7).
+template <int KCAP>
 __global__ __launch_bounds__(kSortThreads) void sel_part_kernel(SelectParams p, const float* nx, const float* nv,
                                                                 const double* stats, int psize, int nparts, int kpad,
                                                                 unsigned long long* out) {
     __shared__ KthShared sh;
     __shared__ unsigned long long keys[kPartMax];
+    __shared__ SetStats ss;
+    __shared__ int sel[KCAP > 0 ? KCAP : 1];
     const int tid = threadIdx.x;
     const int part = blockIdx.x % nparts, sidx = blockIdx.x / nparts;
     const int s = sidx % p.num_seqs, h = sidx / p.num_seqs;
     int st, len;
     seq_bounds(p.cu, s, p.total_len, p.max_seqlen, st, len);
     const int g = h / (p.n_heads / p.n_kv_heads), r = global_range(p, s);
-    double mean[2], sd[2];
     if (stats) {  // written by sel_sums
         const int nsig = 1 + p.n_kv_heads;
-        const double* sx = stats + (int64_t)r * nsig * 2;
-        const double* sv = stats + ((int64_t)r * nsig + 1 + g) * 2;
-        mean[0] = sx[0];
-        sd[0] = sx[1];
-        mean[1] = sv[0];
-        sd[1] = sv[1];
+        if (tid < 2) {
+            const double* x = stats + ((int64_t)r * nsig + (tid ? 1 + g : 0)) * 2;
+            ss.mean[tid] = x[0];
+            ss.sd[tid] = x[1];
+            ss.rsd[tid] = __ddiv_rn(1.0, x[1]);
+        }
+        __syncthreads();
     } else {
-        pair_stats(p, nx, nv, r, g, mean, sd);
+        pair_stats(p, nx, nv, r, g, ss);
     }
-    const KeyFn key = global_key_of(p, nx, nv, st, h, mean[0], sd[0], mean[1], sd[1]);
+    const KeyFn key = global_key_of(p, nx, nv, st, h, ss);
     const int j0 = part * psize;
     const int n = max(0, min(psize, len - j0));
     for (int i = tid; i < n; i += kSortThreads) keys[i] = key(j0 + i);
     __syncthreads();
-    keep_largest(sh, keys, n, kpad, out + ((int64_t)sidx * nparts + part) * kpad, tid);
+    if constexpr (KCAP > 0) write_set(p, sh, keys, n, sel, sidx, tid);
+    else keep_largest(sh, keys, n, kpad, out + ((int64_t)sidx * nparts + part) * kpad, tid);
 }
 
 // merge parts [op*G, op*G+G) of set sidx (G*kpad <= kMergeMax keys): with `out`, keep
@@ -936,22 +984,7 @@ __global__ __launch_bounds__(kSortThreads) void sel_merge_kernel(SelectParams p,
         keep_largest(sh, keys, m, kpad, out + ((int64_t)sidx * nout + op) * kpad, tid);
         return;
     }
-    // the K largest keys: those above the K-th largest, and it when it is a candidate's
-    // key (keys of candidates are distinct; fewer than K candidates leave it 0)
-    const int K = p.k_lmk;
-    const unsigned long long kk = kth_desc(sh, keys, m, K - 1, tid);
-    if (tid == 0) sh.ncand = 0u;
-    __syncthreads();
-    for (int i = tid; i < m; i += kSortThreads) {
-        const unsigned long long kj = keys[i];
-        if (kj > kk || (kj == kk && kk != 0ull))
-            sel[atomicAdd(&sh.ncand, 1u)] = (int)(0xffffffffu - (uint32_t)(kj & 0xffffffffull));
-    }
-    __syncthreads();
-    const int nsel = (int)sh.ncand;
-    int32_t* o = p.lmk_idx + (int64_t)sidx * K;
-    rank_sort_asc<kSelThreads>(sel, nsel, o, tid);
-    for (int i = nsel + tid; i < K; i += kSortThreads) o[i] = -1;
+    write_set(p, sh, keys, m, sel, sidx, tid);
 }
 
 template <int NT, int KCAP>
@@ -1425,8 +1458,18 @@ hipError_t select_launch(const SelectParams& p, void* ws, hipStream_t stream, in
     unsigned long long* ka = (unsigned long long*)w;
     unsigned long long* kb2 = (unsigned long long*)(w + kb);
     const bool stats_written = !parts_own_stats(p);
-    DSALT_LAUNCH("sel_part", sel_part_kernel, dim3(nsets_total * t.nparts), dim3(kSortThreads), 0, stream, p, nx, nv,
-                 stats_written ? stats : nullptr, t.psize, t.nparts, t.kpad, ka);
+    const double* st = stats_written ? stats : nullptr;
+    if (t.nparts == 1) {  // the part writes the set
+        if (p.k_lmk > kSetSlots)
+            DSALT_LAUNCH("sel_part", sel_part_kernel<kMaxLandmarks>, dim3(nsets_total), dim3(kSortThreads), 0, stream, p,
+                         nx, nv, st, t.psize, 1, t.kpad, nullptr);
+        else
+            DSALT_LAUNCH("sel_part", sel_part_kernel<kSetSlots>, dim3(nsets_total), dim3(kSortThreads), 0, stream, p, nx,
+                         nv, st, t.psize, 1, t.kpad, nullptr);
+        return hipGetLastError();
+    }
+    DSALT_LAUNCH("sel_part", sel_part_kernel<0>, dim3(nsets_total * t.nparts), dim3(kSortThreads), 0, stream, p, nx, nv,
+                 st, t.psize, t.nparts, t.kpad, ka);
     // keys per merge block <= kMergeMax
     auto merge = [&](int nin, unsigned long long* out, int nout) {
         if (p.k_lmk > kSetSlots)
