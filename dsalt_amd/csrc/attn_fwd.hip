@@ -207,12 +207,16 @@ __device__ __forceinline__ void band_edge(const AttnParams& p, const RowGroup& R
 // (head, sequence) pairs from which each XCD walks its pairs one at a time (fwd_kernel)
 constexpr int kPairOrderMin = 256;
 
-template <typename T, int D, int BN, int RG, bool TR, bool MS = false, int NW = 4>
+//
+// IP: each block makes its tile's row plan itself (plan_regs, by every wave; head 0's blocks also
+// write it to the plan buffer) instead of reading the one a launch before it wrote.
+template <typename T, int D, int BN, int RG, bool TR, bool MS = false, int NW = 4, bool IP = false>
 __global__ __launch_bounds__(64 * NW, ((sizeof(T) == 2 && D == 64 && RG == 2 && BN == 32) ||
                                        (sizeof(T) == 2 && D == 128 && RG == 1 && BN == 32 && NW == 4 && TR))
                                           ? 4
                                           : 2) void fwd_kernel(AttnParams p) {
     static_assert(!MS || (RG == 1 && !TR), "several sets per block: one row group, inference");
+    static_assert(!IP || (RG == 1 && NW == 4 && !MS), "plan in the block: one plan tile per block");
     static_assert(NW == 4 || (NW == 8 && RG == 1 && !MS), "eight waves: one row group each, one set per block");
     constexpr int NT = 64 * NW;
     constexpr int TPB = RG * NW / 4;  // plan tiles (64 rows) per block
@@ -260,7 +264,12 @@ __global__ __launch_bounds__(64 * NW, ((sizeof(T) == 2 && D == 64 && RG == 2 && 
     int st, len;
     seq_bounds(p.cu, s, p.total_len, p.max_seqlen, st, len);
     const int r0 = b * 64 * TPB;
-    if (r0 >= len) return;
+    if (r0 >= len) {
+        if (IP && h == 0 && wave == 0)  // the plan's entry of a tile past the sequence's end
+            plan_store(plan_regs(p.w, st, len, r0, lane), (int64_t)s * p.n_tiles + b, lane,
+                       PlanOut{p.plan_perm, p.plan_bounds, p.tile_wmax});
+        return;
+    }
     const int kvh = h / (p.n_heads / p.n_kv_heads);
     const int set = p.block_size ? r0 / p.block_size : 0;
     const int K = p.k_lmk;
@@ -301,16 +310,27 @@ __global__ __launch_bounds__(64 * NW, ((sizeof(T) == 2 && D == 64 && RG == 2 && 
     const int64_t tile0 = (int64_t)s * p.n_tiles + (int64_t)b * TPB;
     const int ntl = min(TPB, p.n_tiles - b * TPB);
     int blo = 0x7fffffff, bhi = -1, blmax = (int)0x80000000;
-    if (lane < 4 * ntl) {
-        const int* bnd = p.plan_bounds + tile0 * 16 + lane * 4;
-        blo = bnd[0];
-        blmax = bnd[1];
-        bhi = bnd[2];
-    }
     PlanLoad pl[RG];
+    if constexpr (IP) {
+        const PlanRegs r = plan_regs(p.w, st, len, r0, lane);
+        if (h == 0 && uw == 0) plan_store(r, tile0, lane, PlanOut{p.plan_perm, p.plan_bounds, p.tile_wmax});
+        blo = r.lo;
+        blmax = r.lomax;
+        bhi = r.hi;
+        pl[0] = PlanLoad{__builtin_amdgcn_readlane(r.lo, uw * 16), __builtin_amdgcn_readlane(r.lomax, uw * 16),
+                         __builtin_amdgcn_readlane(r.hi, uw * 16), __builtin_amdgcn_readlane(r.himin, uw * 16),
+                         __shfl(r.perm, uw * 16 + (lane & 15))};
+    } else {
+        if (lane < 4 * ntl) {
+            const int* bnd = p.plan_bounds + tile0 * 16 + lane * 4;
+            blo = bnd[0];
+            blmax = bnd[1];
+            bhi = bnd[2];
+        }
 #pragma unroll
-    for (int u = 0; u < RG; ++u) pl[u] = plan_load(p, tile0, ntl, group_of<RG>(uw, u), lane);
-    __builtin_amdgcn_sched_barrier(0);  // every group's plan load issued before any is used
+        for (int u = 0; u < RG; ++u) pl[u] = plan_load(p, tile0, ntl, group_of<RG>(uw, u), lane);
+        __builtin_amdgcn_sched_barrier(0);  // every group's plan load issued before any is used
+    }
     RowGroup rg[RG];
 #pragma unroll
     for (int u = 0; u < RG; ++u) plan_rows(pl[u], ntl, group_of<RG>(uw, u), r0, len, rg[u]);
@@ -717,15 +737,33 @@ static int fwd_variant(const AttnParams& p) {
     return !TR && tiles >= kW8Tiles ? p.variant | DSALT_VARIANT_FWD_8W : p.variant;
 }
 
+// Calls of up to kInlineTiles 64-row tiles (x heads) make the plan in the attention's own blocks: the
+// launch before costs its own latency, a plan per block and head under a microsecond of each
+// round of blocks.  Plan and forward, us (graph replay, so without the launch's 3 us on the host):
+// 32 tiles 12.1 -> 10.1, 512 14.7 -> 13.3, 1024 19.7 -> 19.1, 1375 39.2 -> 39.7; head_dim 128: 256
+// tiles 14.5 -> 12.4, 1024 24.7 -> 22.9, 8192 125 -> 136; float32: 512 29.1 -> 26.8, 2048 72.8 -> 74.5.
+constexpr int64_t kInlineTiles = 1024;
+
 template <typename T, int D, bool TR>
-static void fwd_run(const AttnParams& p, hipStream_t stream) {
+static hipError_t fwd_run(const AttnParams& p, bool plan_ready, hipStream_t stream) {
     constexpr int BN = FwdShape<T, D>::BN;
     const int variant = fwd_variant<T, D, TR>(p);
+    constexpr int kTilings = DSALT_VARIANT_FWD_BN32 | DSALT_VARIANT_FWD_RG2 | DSALT_VARIANT_FWD_BN64 | DSALT_VARIANT_FWD_8W;
+    if (!plan_ready) {
+        const int64_t tiles = (int64_t)p.total_len * p.n_heads / 64;
+        if (!(variant & kTilings) && p.block_size % 64 == 0 && p.k_lmk <= kSetSlots && tiles <= kInlineTiles) {
+            DSALT_LAUNCH("attn_fwd", (fwd_kernel<T, D, BN, 1, TR, false, 4, true>),
+                         dim3(p.n_heads * p.num_seqs * p.n_tiles), dim3(256), 0, stream, p);
+            return hipGetLastError();
+        }
+        const hipError_t e = plan_launch(p, stream);
+        if (e != hipSuccess) return e;
+    }
     if constexpr (!TR) {
         if (p.block_size % 64 || p.k_lmk > kSetSlots) {
             DSALT_LAUNCH("attn_fwd", (fwd_kernel<T, D, BN, 1, false, true>), dim3(p.n_heads * p.num_seqs * p.n_tiles),
                          dim3(256), 0, stream, p);
-            return;
+            return hipGetLastError();
         }
     }
     if constexpr (sizeof(T) == 2) {
@@ -736,11 +774,11 @@ static void fwd_run(const AttnParams& p, hipStream_t stream) {
             if (rg2) {
                 if (bn32) DSALT_LAUNCH("attn_fwd", (fwd_kernel<T, D, 32, 2, TR>), dim3(total), dim3(256), 0, stream, p);
                 else DSALT_LAUNCH("attn_fwd", (fwd_kernel<T, D, BN, 2, TR>), dim3(total), dim3(256), 0, stream, p);
-                return;
+                return hipGetLastError();
             }
             if (bn32) {
                 DSALT_LAUNCH("attn_fwd", (fwd_kernel<T, D, 32, 1, TR>), dim3(total), dim3(256), 0, stream, p);
-                return;
+                return hipGetLastError();
             }
         } else if constexpr (!TR) {  // head_dim 128 (inference shapes)
             // two row groups keep 32-key chunks (with 64-key chunks they would spill at 256 VGPRs)
@@ -749,41 +787,34 @@ static void fwd_run(const AttnParams& p, hipStream_t stream) {
             if (w8) {
                 DSALT_LAUNCH("attn_fwd", (fwd_kernel<T, D, BN, 1, TR, false, 8>),
                              dim3(p.n_heads * p.num_seqs * ceil_div(p.n_tiles, 2)), dim3(512), 0, stream, p);
-                return;
+                return hipGetLastError();
             }
             if (rg2) {
                 DSALT_LAUNCH("attn_fwd", (fwd_kernel<T, D, BN, 2, TR>), dim3(total), dim3(256), 0, stream, p);
-                return;
+                return hipGetLastError();
             }
             if (bn64) {
                 DSALT_LAUNCH("attn_fwd", (fwd_kernel<T, D, 64, 1, TR>), dim3(total), dim3(256), 0, stream, p);
-                return;
+                return hipGetLastError();
             }
         }
     }
     const int total = p.n_heads * p.num_seqs * p.n_tiles;
     DSALT_LAUNCH("attn_fwd", (fwd_kernel<T, D, BN, 1, TR>), dim3(total), dim3(256), 0, stream, p);
+    return hipGetLastError();
 }
 
 template <typename T>
 static hipError_t fwd_dispatch(AttnParams p, bool plan_ready, hipStream_t stream) {
     if (p.n_heads * p.num_seqs * p.n_tiles == 0) return hipSuccess;
-    if (!plan_ready) {
-        const hipError_t e = plan_launch(p, stream);
-        if (e != hipSuccess) return e;
-    }
     // without a soft edge every band key's bias is 0: the training forward is the operator over
     // the integer windows, in the operator's tiling
     const bool tr = p.w_cont != nullptr && p.edge > 0.f;
     if (!tr) p.w_cont = nullptr;
     if (p.head_dim == 64) {
-        if (tr) fwd_run<T, 64, true>(p, stream);
-        else fwd_run<T, 64, false>(p, stream);
-    } else {
-        if (tr) fwd_run<T, 128, true>(p, stream);
-        else fwd_run<T, 128, false>(p, stream);
+        return tr ? fwd_run<T, 64, true>(p, plan_ready, stream) : fwd_run<T, 64, false>(p, plan_ready, stream);
     }
-    return hipGetLastError();
+    return tr ? fwd_run<T, 128, true>(p, plan_ready, stream) : fwd_run<T, 128, false>(p, plan_ready, stream);
 }
 
 // training variant: integer windows floor(w~) + 1 (w~ below 0 as 0, at most max_seqlen);

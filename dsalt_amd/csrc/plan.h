@@ -19,6 +19,51 @@ struct PlanOut {
     int* wmax;       // [S * n_tiles]
 };
 
+// The plan of one tile in the registers of a wave (every lane calls it; lane l holds sorted
+// position l): the row offset at that position, its 16-row group's bounds, and the tile's largest
+// window.  The forward's blocks compute it themselves where a call is too small to hide the
+// plan's own launch.
+struct PlanRegs {
+    int perm, lo, lomax, hi, himin, wmax;
+};
+__device__ __forceinline__ PlanRegs plan_regs(const int32_t* w, int st, int len, int r0, int l) {
+    const int i = r0 + l;
+    int lo = 0x7fffffff, wcl = 0;
+    if (i < len) {
+        const int wi = max(w[st + i], 1);
+        lo = max(i - wi + 1, 0);
+        wcl = min(wi, len);
+    }
+    int rank = 0;  // by (lo, row)
+#pragma unroll 8
+    for (int j = 0; j < 64; ++j) {
+        const int jlo = __builtin_amdgcn_readlane(lo, j);
+        rank += (jlo < lo || (jlo == lo && j < l)) ? 1 : 0;
+    }
+    PlanRegs r;
+    r.perm = __builtin_amdgcn_ds_permute(rank * 4, l);
+    const bool rv = r0 + r.perm < len;
+    const int slo = __shfl(lo, r.perm);
+    r.lo = row_min16(rv ? slo : 0x7fffffff);
+    r.lomax = row_max16(rv ? slo : (int)0x80000000);
+    r.hi = row_max16(rv ? r0 + r.perm : -1);
+    r.himin = row_min16(rv ? r0 + r.perm : 0x7fffffff);
+    r.wmax = wave_max(wcl);
+    return r;
+}
+// writes it where row_plan_tile would (one wave)
+__device__ __forceinline__ void plan_store(const PlanRegs& r, int64_t tile, int l, const PlanOut& o) {
+    o.perm[tile * 64 + l] = (uint8_t)r.perm;
+    if ((l & 15) == 0) {
+        int* b = o.bounds + (tile * 4 + (l >> 4)) * 4;
+        b[0] = r.lo;
+        b[1] = r.lomax;
+        b[2] = r.hi;
+        b[3] = r.himin;
+    }
+    if (l == 0) o.wmax[tile] = r.wmax;
+}
+
 // One wave (lane l) plans tile `tile` (= s * n_tiles + t) when `active`; sp, slo: 64 ints
 // of LDS each, private to the wave.  Every thread of the block must call it once (one
 // block barrier inside); nothing is written for an inactive tile.

@@ -58,6 +58,8 @@ def _dense(q, k, v, w, cu, idx, block, heads):
 
 
 @pytest.mark.parametrize("lens,H,G,D,dt,block", [
+    ([8190], 8, 8, 64, torch.bfloat16, 0),                # the blocks make their own row plan
+    ([8200], 8, 8, 64, torch.bfloat16, 0),                # past 1024 tiles a launch before them does
     ([6143], 16, 4, 64, torch.bfloat16, 0),               # below 1536 tiles of 64 rows
     ([6145], 16, 16, 64, torch.bfloat16, 0),              # above, an odd number of tiles
     ([4097, 1, 2050, 190], 16, 2, 64, torch.float16, 0),  # ragged
@@ -75,6 +77,23 @@ def test_forward_tiling_by_size(lens, H, G, D, dt, block):
     heads = sorted({0, H // 2 + 1, H - 1})
     ref = _dense(q, k, v, w, cu, idx, block, heads)
     assert (out[:, heads].float() - ref).abs().max() <= 3 * UNIT[dt] * v.float().abs().max()
+
+
+@pytest.mark.parametrize("lens,H", [([8190], 8), ([8200], 8), ([700, 0, 1, 64, 65], 4), ([700, 0, 1, 64, 65], 160)])
+@pytest.mark.parametrize("D,dt", [(64, torch.bfloat16), (128, torch.float16), (64, torch.float32)])
+def test_plan_made_by_the_blocks(lens, H, D, dt):
+    """The row plan of the attention's own blocks (small calls) is the selection's, byte for byte,
+    tiles past a sequence's end included, and the output that of a plan made before."""
+    q, k, v, w, cu, idx = _inputs(lens, H, 2, D, 9, 150, dt, seed=3)
+    h, alpha = torch.randn(q.shape[0], 64, device=DEV).to(dt), torch.full((H,), 0.5, device=DEV)
+    made, given = (ops.new_plan(q, k, cu, idx, max_seqlen=max(lens)).fill_(0) for _ in range(2))
+    ops.select_landmarks(h, v, alpha, w, cu, 4, max_seqlen=max(lens), plan=given)
+    a = ops.attention_forward(q, k, v, w, cu, idx, max_seqlen=max(lens), plan=made)
+    b = ops.attention_forward(q, k, v, w, cu, idx, max_seqlen=max(lens), plan=given, plan_ready=True)
+    n = sum(x * y for x, y in ((64, 1), (16, 4), (1, 4))) * len(lens) * -(-max(lens) // 64)
+    assert torch.equal(made, given) and made.numel() >= n
+    T = int(cu[-1])
+    assert torch.equal(a[0][:T], b[0][:T]) and torch.equal(a[1][:T], b[1][:T])
 
 
 @pytest.mark.parametrize("lens,H,G,D,K,dt", [
@@ -120,3 +139,27 @@ def test_grouped_gradients_equal_those_of_repeated_heads(lens, H, G, D, K, dt, t
     again = run(k, v)
     for a, b in zip(got, again):
         assert torch.equal(a, b)  # one writer per element, sums in a fixed order
+
+
+@pytest.mark.parametrize("lens,K", [([2047], 32), ([2048], 600), ([2049], 32), ([1, 0, 30, 2048], 40), ([5, 3], 2048),
+                                    ([2048, 2049, 700], 512), ([1500], 1)])
+@pytest.mark.parametrize("scope", [ops.STATS_PACKED, ops.STATS_SEQUENCE])
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+def test_selection_of_one_part_sets_bit_exact(lens, K, scope, dt):
+    """Sequences of up to 2048 tokens are selected by one block a set, longer ones by parts and
+    merges: the oracle's indices on both sides."""
+    import numpy as np
+
+    from oracle import select as OS
+    from tests.helpers import bits, oracle_dtype
+    g = torch.Generator().manual_seed(sum(lens) + K)
+    T, H, G = sum(lens), 4, 2
+    h, v = torch.randn(T, 96, generator=g).to(dt), torch.randn(T, G, 64, generator=g).to(dt)
+    v[torch.rand(T, generator=g) < 0.1] = 0  # ties
+    w = torch.randint(1, 200, (T,), generator=g, dtype=torch.int32)
+    cu = torch.tensor([0] + list(np.cumsum(lens)), dtype=torch.int32)
+    alpha = torch.tensor([0.0, 0.3, 0.7, 1.0])
+    idx = ops.select_landmarks(h.to(DEV), v.to(DEV), alpha.to(DEV), w.to(DEV), cu.to(DEV), K, max_seqlen=max(lens),
+                               stats_scope=scope)
+    ref = OS.select(bits(h), bits(v), alpha.numpy(), w.numpy(), cu.numpy(), K, oracle_dtype(dt), stats_scope=scope)
+    assert np.array_equal(idx.cpu().numpy(), ref)
