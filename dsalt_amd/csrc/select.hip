@@ -429,11 +429,12 @@ constexpr int kKthCand = 64;       // radix passes of kth_desc stop once the bin
 template <int NT_, int KCAP>
 struct TopkShared {
     static constexpr int NT = NT_;
-    uint32_t hist[NT_ / kWave][256];
+    __attribute__((aligned(16))) uint32_t hist[NT_ / kWave][256];
     unsigned long long border[kBorderCap > kSample ? kBorderCap : kSample];
     int sel[KCAP];
     unsigned long long cand[kKthCand];
     unsigned long long kth;
+    uint32_t wsum[NT_ / kWave];
     uint32_t total;
     int digit;
     uint32_t above;
@@ -445,39 +446,87 @@ struct TopkShared {
 // LDS of kth_desc alone (the global top-k parts and merges)
 struct KthShared {
     static constexpr int NT = kSelThreads;
-    uint32_t hist[kSelWaves][256];
+    __attribute__((aligned(16))) uint32_t hist[kSelWaves][256];
     unsigned long long cand[kKthCand];
     unsigned long long kth;
+    uint32_t wsum[kSelWaves];
     int digit;
     uint32_t above;
     uint32_t ncand;
 };
 
-// The r-th largest (0-based) of the n keys a[0..n) in LDS, for the whole block: radix
-// passes over 8-bit digits from the top (per-wave LDS histograms, as in the selection
-// below) narrow the keys to one digit prefix until at most kKthCand remain; those are
-// gathered and the answer is the candidate c with #{> c} <= r < #{>= c} (equal keys all
-// qualify and write the same value).  Exact for any keys; replaces a full sort where only
-// one order statistic is needed.
+// The r-th largest (0-based) of the n keys a[0..n) in LDS, for the whole block: passes over
+// digits from the top narrow the keys to one digit prefix until at most kKthCand remain; those
+// are gathered and the answer is the candidate c with #{> c} <= r < #{>= c} (equal keys all
+// qualify and write the same value).  Exact for any keys; replaces a full sort where only one
+// order statistic is needed.  The first digit has 4 bins a thread (10 to 12 bits: sign, exponent
+// and one to three mantissa bits of the score), which usually leaves so few keys that no second
+// pass follows; an 8-bit first digit holds whole octaves of scores and never did.  The
+// zero keys of non-candidates are left out throughout (the answer is 0 when fewer than r + 1
+// other keys exist).
 template <class Sh>
 __device__ unsigned long long kth_desc(Sh& sh, const unsigned long long* a, int n, int r, int tid) {
     const int wave = tid >> 6, lane = tid & 63;
+    constexpr int NW = Sh::NT / kWave, B0 = Sh::NT == 1024 ? 12 : Sh::NT == 512 ? 11 : 10;
+    static_assert((1 << B0) == 4 * Sh::NT, "four bins of the first digit per thread");
+    uint32_t* const bins = &sh.hist[0][0];
     unsigned long long prefix = 0ull;
     int plen = 0;
     uint32_t rem = (uint32_t)r;
-    for (;;) {
-        for (int i = tid; i < (Sh::NT / kWave) * 256; i += Sh::NT) (&sh.hist[0][0])[i] = 0u;
+    for (int i = tid; i < 4 * Sh::NT; i += Sh::NT) bins[i] = 0u;
+    if (tid == 0) sh.digit = -1;
+    __syncthreads();
+    for (int i = tid; i < n; i += Sh::NT) {
+        const unsigned long long k = a[i];
+        if (k) atomicAdd(&bins[(uint32_t)(k >> (64 - B0))], 1u);
+    }
+    __syncthreads();
+    {
+        const uint4 c4 = *(const uint4*)(bins + 4 * tid);
+        const uint32_t cs[4] = {c4.x, c4.y, c4.z, c4.w};
+        const uint32_t loc = cs[0] + cs[1] + cs[2] + cs[3];
+        uint32_t suf = loc;  // over this and the higher lanes of the wave
+        for (int off = 1; off < 64; off <<= 1) {
+            const uint32_t o = __shfl_down(suf, off, 64);
+            if (lane + off < 64) suf += o;
+        }
+        if (lane == 0) sh.wsum[wave] = suf;
         __syncthreads();
-        const int shift = 56 - plen;
+        uint32_t above = suf - loc;
+        for (int w2 = wave + 1; w2 < NW; ++w2) above += sh.wsum[w2];
+#pragma unroll
+        for (int b = 3; b >= 0; --b) {
+            if (above <= rem && rem < above + cs[b]) {
+                sh.digit = 4 * tid + b;
+                sh.above = above;
+                sh.ncand = cs[b];
+            }
+            above += cs[b];
+        }
+    }
+    __syncthreads();
+    if (sh.digit < 0) {  // at most r keys are not zero
+        __syncthreads();
+        return 0ull;
+    }
+    rem -= sh.above;
+    prefix = (unsigned long long)sh.digit;
+    plen = B0;
+    uint32_t inbin = sh.ncand;
+    __syncthreads();
+    while (inbin > (uint32_t)kKthCand) {
+        for (int i = tid; i < NW * 256; i += Sh::NT) bins[i] = 0u;
+        __syncthreads();
+        const int nb = min(8, 64 - plen), shift = 64 - plen - nb;
         for (int i = tid; i < n; i += Sh::NT) {
             const unsigned long long k = a[i];
-            if (plen > 0 && (k >> (64 - plen)) != prefix) continue;
-            atomicAdd(&sh.hist[wave][(uint32_t)(k >> shift) & 255u], 1u);
+            if (!k || (k >> (64 - plen)) != prefix) continue;
+            atomicAdd(&sh.hist[wave][(uint32_t)(k >> shift) & ((1u << nb) - 1u)], 1u);
         }
         __syncthreads();
         if (tid < 256) {
             uint32_t c = 0;
-            for (int w2 = 0; w2 < (Sh::NT / kWave); ++w2) c += sh.hist[w2][tid];
+            for (int w2 = 0; w2 < NW; ++w2) c += sh.hist[w2][tid];
             sh.hist[0][tid] = c;
         }
         __syncthreads();
@@ -502,19 +551,18 @@ __device__ unsigned long long kth_desc(Sh& sh, const unsigned long long* a, int 
         }
         __syncthreads();
         const int d = sh.digit;
-        const uint32_t inbin = sh.hist[0][d];
+        inbin = sh.hist[0][d];
         rem -= sh.above;
-        prefix = (prefix << 8) | (unsigned long long)d;
-        plen += 8;
+        prefix = (prefix << nb) | (unsigned long long)d;
+        plen += nb;
         if (plen == 64) return prefix;  // every bit fixed
-        if (inbin <= (uint32_t)kKthCand) break;
         __syncthreads();  // hist and digit are rewritten by the next pass
     }
     if (tid == 0) sh.ncand = 0u;
     __syncthreads();
     for (int i = tid; i < n; i += Sh::NT) {
         const unsigned long long k = a[i];
-        if ((k >> (64 - plen)) == prefix) sh.cand[atomicAdd(&sh.ncand, 1u)] = k;
+        if (k && (k >> (64 - plen)) == prefix) sh.cand[atomicAdd(&sh.ncand, 1u)] = k;
     }
     __syncthreads();
     const int m = (int)sh.ncand;
