@@ -694,13 +694,18 @@ __global__ __launch_bounds__(64 * NW, ((sizeof(T) == 2 && D == 64 && RG == 2 && 
     for (int u = 0; u < RG; ++u) {
         const float l_tot = kHalf ? lacc[u][0] : sum_g4(l_run[u]);
         const int vi = rg[u].valid ? rg[u].i : -1;
-        SR::run(stage, acc[u], rg[u].valid ? 1.0f / l_tot : 0.f, lane, [&](int rr) {
+        const float inv = rg[u].valid ? 1.0f / l_tot : 0.f;
+        auto row16 = [&](int rr) {
             const int ir = __shfl(vi, rr);
             return ir >= 0 ? o0 + (int64_t)ir * p.o_st : (T*)nullptr;
-        }, [&](int rr) {
-            const int ir = p.out32 ? __shfl(vi, rr) : -1;
-            return ir >= 0 ? p.out32 + ((int64_t)(st + ir) * p.n_heads + h) * D : (float*)nullptr;
-        });
+        };
+        if (kHalf && p.out32)
+            SR::run(stage, acc[u], inv, lane, row16, [&](int rr) {
+                const int ir = __shfl(vi, rr);
+                return ir >= 0 ? p.out32 + ((int64_t)(st + ir) * p.n_heads + h) * D : (float*)nullptr;
+            });
+        else
+            SR::run(stage, acc[u], inv, lane, row16);
         if (rg[u].valid && g == 0) p.lse_out[(int64_t)(st + rg[u].i) * p.n_heads + h] = m_run[u] * p.scale + __logf(l_tot);
     }
 }
