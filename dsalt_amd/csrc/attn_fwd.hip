@@ -716,30 +716,38 @@ __global__ __launch_bounds__(64 * NW, ((sizeof(T) == 2 && D == 64 && RG == 2 && 
 // row groups per wave (FWD_RG2, same condition) or 64-key chunks instead of 32 (FWD_BN64;
 // ignored with FWD_RG2);
 // fp32 takes its single compiled tiling.  With no forward bit set the call picks by its work
-// in 64-row tiles, tokens x heads / 64 (one call, plan included, against the 64-row tiling of
-// 64-key, at head_dim 128 32-key, chunks; windows up to 64 .. 512, 16 .. 256 landmarks):
-//   head_dim 64: FWD_RG2 | FWD_BN32 from kRg2Tiles on.  The 128-row blocks read each K and V^T
-//     operand from LDS once for 32 rows (the 64-row tiling reads 1 KB of LDS per MFMA), but below
-//     that there are too few of them: 1024 tiles 1.04-1.07x the time, 1536 0.90-0.96x, 2048
-//     0.86-0.95x, 8192 0.80-0.82x (16 heads x 32768, windows up to 512: 153.5 -> 123.1 us);
+// in 64-row tiles, tokens x heads / 64, among tilings whose outputs are the same bit for bit: equal
+// key chunks on the same boundaries, so the same running maxima and roundings of P (32-key chunks at
+// head_dim 64 round P against other maxima, 2.18e-3 against 2.13e-3 from the float64 result at
+// 16 heads x 32768, and are left to the caller's bit).  Against the 64-row tiling, row plan given,
+// windows up to 64 .. 512, 16 .. 256 landmarks:
+//   head_dim 64: FWD_RG2 from kRg2Tiles on, for sequences of kRg2Len tokens on average.  The 128-row
+//     blocks read each K and V^T operand from LDS once for 32 rows (the 64-row tiling reads 1 KB of
+//     LDS per MFMA), but there are fewer of them: 2048 tiles 1.03-1.06x the time, 4096 0.93-1.01x, 6144
+//     0.93-0.99x, 8192 0.91-0.99x, 32768 0.89-0.92x (16 heads x 32768, windows up to 512: 157.4 ->
+//     146.1 us).  Short sequences leave half of a block without rows: 512 to 700 tokens 0.96-1.02x,
+//     150 to 320 1.05-1.11x, 64 1.22x;
 //   head_dim 128: FWD_8W from kW8Tiles on, where staging the key chunks bounds the kernel: 32768
 //     tiles 0.945-0.997x (16 heads x 131072, 256 landmarks: 1130 -> 1077 us); 8192 tiles
 //     0.93-1.12x and 2048 0.96-1.07x (slower for windows below 512), so these keep four waves.
-// The training variant takes the same line (head_dim 64: 1536 tiles 0.91-0.98x, 4096 0.85-0.91x,
-// 8192 182.2 -> 154.9 us) and has no eight-wave tiling.
+// The training variant keeps 64-row blocks: its two row groups are held to too few registers
+// (1.13-1.26x from 1536 tiles on).
 // Sets of more than kSetSlots landmarks, and
 // block-causal sets of a block_size that is not a multiple of 64, take the default tiling's
 // wide instantiation (variant bits ignored).
-constexpr int64_t kRg2Tiles = 1536, kW8Tiles = 16384;
+constexpr int64_t kRg2Tiles = 6144, kRg2Len = 1024, kW8Tiles = 16384;
 
 // the forward tiling bits the call runs with: its own, or the rule's when it names none
 template <typename T, int D, bool TR>
 static int fwd_variant(const AttnParams& p) {
     constexpr int kFwdBits = DSALT_VARIANT_FWD_BN32 | DSALT_VARIANT_FWD_RG2 | DSALT_VARIANT_FWD_BN64 | DSALT_VARIANT_FWD_8W;
-    if (sizeof(T) != 2 || (p.variant & kFwdBits) || p.block_size % 128) return p.variant;
+    if (sizeof(T) != 2 || TR || (p.variant & kFwdBits) || p.block_size % 128) return p.variant;
     const int64_t tiles = (int64_t)p.total_len * p.n_heads / 64;
-    if (D == 64) return tiles >= kRg2Tiles ? p.variant | DSALT_VARIANT_FWD_RG2 | DSALT_VARIANT_FWD_BN32 : p.variant;
-    return !TR && tiles >= kW8Tiles ? p.variant | DSALT_VARIANT_FWD_8W : p.variant;
+    if (D == 64) {
+        const bool pairs = tiles >= kRg2Tiles && p.total_len >= kRg2Len * p.num_seqs;
+        return pairs ? p.variant | DSALT_VARIANT_FWD_RG2 : p.variant;
+    }
+    return tiles >= kW8Tiles ? p.variant | DSALT_VARIANT_FWD_8W : p.variant;
 }
 
 // Calls of up to kInlineTiles 64-row tiles (x heads) make the plan in the attention's own blocks: the
