@@ -137,6 +137,7 @@ SIGNATURES = {
     "dsalt_select_with_border_cap": ([ctypes.POINTER(SelectArgs), _vp, ctypes.c_int], ctypes.c_int),
     "dsalt_select_workspace_bytes_cap": ([ctypes.POINTER(SelectArgs), ctypes.c_int], _sz),
     "dsalt_plan_bytes": ([ctypes.POINTER(Problem)], _sz),
+    "dsalt_fwd_tile": ([ctypes.POINTER(Problem), _i32] + [ctypes.POINTER(_i32)] * 3, ctypes.c_int),
     "dsalt_fwd_workspace_bytes": ([ctypes.POINTER(FwdArgs)], _sz),
     "dsalt_fwd": ([ctypes.POINTER(FwdArgs), _vp], ctypes.c_int),
     "dsalt_fwd_noalloc": ([ctypes.POINTER(FwdArgs), _vp], ctypes.c_int),

@@ -136,6 +136,13 @@ hipError_t plan_launch(const AttnParams& p, hipStream_t stream);
 // plan: a caller buffer of plan_bytes() that receives the row plan, or null (workspace);
 // plan_ready: the buffer already holds the plan of these rows (not recomputed)
 hipError_t fwd_launch(AttnParams p, void* ws, void* plan, bool plan_ready, hipStream_t stream);
+// the forward's tiling: query rows, keys a chunk and waves of a block, and whether a block takes
+// several or large landmark sets
+struct FwdTile {
+    int rows, keys, waves;
+    bool multi;
+};
+FwdTile fwd_tile(const AttnParams& p, bool train);
 // training variant: integer windows floor(w~) + 1 written into `w_int` ([T] int32)
 hipError_t train_windows_launch(const AttnParams& p, int* w_int, hipStream_t stream);
 // plan_given: the caller supplies the row plan (no room for it in the workspace)

@@ -714,8 +714,9 @@ __global__ __launch_bounds__(64 * NW, ((sizeof(T) == 2 && D == 64 && RG == 2 && 
 // (FWD_BN32) and two 16-row groups per wave (FWD_RG2, 128 rows per block: the block must
 // stay within one landmark set, block_size a multiple of 128); for 16-bit head_dim 128, two
 // row groups per wave (FWD_RG2, same condition) or 64-key chunks instead of 32 (FWD_BN64;
-// ignored with FWD_RG2);
-// fp32 takes its single compiled tiling.  With no forward bit set the call picks by its work
+// ignored with FWD_RG2).  The bit of the chunk length a head_dim has anyway (FWD_BN64 at 64,
+// FWD_BN32 at 128) asks for its 64-row blocks at any size; fp32 takes its single compiled
+// tiling.  With no forward bit set the call picks by its work
 // in 64-row tiles, tokens x heads / 64, among tilings whose outputs are the same bit for bit: equal
 // key chunks on the same boundaries, so the same running maxima and roundings of P (32-key chunks at
 // head_dim 64 round P against other maxima, 2.18e-3 against 2.13e-3 from the float64 result at
@@ -732,22 +733,34 @@ __global__ __launch_bounds__(64 * NW, ((sizeof(T) == 2 && D == 64 && RG == 2 && 
 //     0.93-1.12x and 2048 0.96-1.07x (slower for windows below 512), so these keep four waves.
 // The training variant keeps 64-row blocks: its two row groups are held to too few registers
 // (1.13-1.26x from 1536 tiles on).
-// Sets of more than kSetSlots landmarks, and
-// block-causal sets of a block_size that is not a multiple of 64, take the default tiling's
-// wide instantiation (variant bits ignored).
+// Sets of more than kSetSlots landmarks, and block-causal sets of a block_size that is not a
+// multiple of 64, take the default tiling's wide instantiation (variant bits ignored).
 constexpr int64_t kRg2Tiles = 6144, kRg2Len = 1024, kW8Tiles = 16384;
 
-// the forward tiling bits the call runs with: its own, or the rule's when it names none
-template <typename T, int D, bool TR>
-static int fwd_variant(const AttnParams& p) {
-    constexpr int kFwdBits = DSALT_VARIANT_FWD_BN32 | DSALT_VARIANT_FWD_RG2 | DSALT_VARIANT_FWD_BN64 | DSALT_VARIANT_FWD_8W;
-    if (sizeof(T) != 2 || TR || (p.variant & kFwdBits) || p.block_size % 128) return p.variant;
+FwdTile fwd_tile(const AttnParams& p, bool train) {
+    const bool half = p.dtype != DSALT_DTYPE_F32;
+    FwdTile t = {64, p.head_dim == 64 ? (half ? 64 : 32) : (half ? 32 : 16), 4, p.block_size % 64 != 0 || p.k_lmk > kSetSlots};
+    if (t.multi || !half) return t;
+    const bool bn32 = p.variant & DSALT_VARIANT_FWD_BN32, bn64 = p.variant & DSALT_VARIANT_FWD_BN64;
+    const bool rg2 = p.variant & DSALT_VARIANT_FWD_RG2, w8 = p.variant & DSALT_VARIANT_FWD_8W;
+    const bool chosen = bn32 || bn64 || rg2 || w8;
+    const bool whole = p.block_size % 128 == 0;  // 128-row blocks stay within one set
     const int64_t tiles = (int64_t)p.total_len * p.n_heads / 64;
-    if (D == 64) {
-        const bool pairs = tiles >= kRg2Tiles && p.total_len >= kRg2Len * p.num_seqs;
-        return pairs ? p.variant | DSALT_VARIANT_FWD_RG2 : p.variant;
+    if (p.head_dim == 64) {
+        const bool by_size = !train && tiles >= kRg2Tiles && p.total_len >= kRg2Len * p.num_seqs;
+        if (whole && (rg2 || (!chosen && by_size))) t.rows = 128;
+        if (bn32) t.keys = 32;
+    } else if (!train) {
+        if (whole && (w8 || (!chosen && tiles >= kW8Tiles))) {
+            t.rows = 128;
+            t.waves = 8;
+        } else if (whole && rg2) {
+            t.rows = 128;  // with 64-key chunks two row groups would spill at 256 VGPRs
+        } else if (bn64) {
+            t.keys = 64;
+        }
     }
-    return tiles >= kW8Tiles ? p.variant | DSALT_VARIANT_FWD_8W : p.variant;
+    return t;
 }
 
 // Calls of up to kInlineTiles 64-row tiles (x heads) make the plan in the attention's own blocks: the
@@ -760,60 +773,45 @@ constexpr int64_t kInlineTiles = 1024;
 template <typename T, int D, bool TR>
 static hipError_t fwd_run(const AttnParams& p, bool plan_ready, hipStream_t stream) {
     constexpr int BN = FwdShape<T, D>::BN;
-    const int variant = fwd_variant<T, D, TR>(p);
-    constexpr int kTilings = DSALT_VARIANT_FWD_BN32 | DSALT_VARIANT_FWD_RG2 | DSALT_VARIANT_FWD_BN64 | DSALT_VARIANT_FWD_8W;
+    const FwdTile t = fwd_tile(p, TR);
+    const dim3 grid(p.n_heads * p.num_seqs * ceil_div(p.n_tiles, t.rows / 64)), block(64 * t.waves);
     if (!plan_ready) {
         const int64_t tiles = (int64_t)p.total_len * p.n_heads / 64;
-        if (!(variant & kTilings) && p.block_size % 64 == 0 && p.k_lmk <= kSetSlots && tiles <= kInlineTiles) {
-            DSALT_LAUNCH("attn_fwd", (fwd_kernel<T, D, BN, 1, TR, false, 4, true>),
-                         dim3(p.n_heads * p.num_seqs * p.n_tiles), dim3(256), 0, stream, p);
+        if (t.rows == 64 && t.keys == BN && !t.multi && tiles <= kInlineTiles) {
+            DSALT_LAUNCH("attn_fwd", (fwd_kernel<T, D, BN, 1, TR, false, 4, true>), grid, block, 0, stream, p);
             return hipGetLastError();
         }
         const hipError_t e = plan_launch(p, stream);
         if (e != hipSuccess) return e;
     }
     if constexpr (!TR) {
-        if (p.block_size % 64 || p.k_lmk > kSetSlots) {
-            DSALT_LAUNCH("attn_fwd", (fwd_kernel<T, D, BN, 1, false, true>), dim3(p.n_heads * p.num_seqs * p.n_tiles),
-                         dim3(256), 0, stream, p);
+        if (t.multi) {
+            DSALT_LAUNCH("attn_fwd", (fwd_kernel<T, D, BN, 1, false, true>), grid, block, 0, stream, p);
             return hipGetLastError();
         }
     }
-    if constexpr (sizeof(T) == 2) {
-        const bool rg2 = (variant & DSALT_VARIANT_FWD_RG2) != 0 && (p.block_size == 0 || p.block_size % 128 == 0);
-        const int total = p.n_heads * p.num_seqs * ceil_div(p.n_tiles, rg2 ? 2 : 1);
-        if constexpr (D == 64) {
-            const bool bn32 = (variant & DSALT_VARIANT_FWD_BN32) != 0;
-            if (rg2) {
-                if (bn32) DSALT_LAUNCH("attn_fwd", (fwd_kernel<T, D, 32, 2, TR>), dim3(total), dim3(256), 0, stream, p);
-                else DSALT_LAUNCH("attn_fwd", (fwd_kernel<T, D, BN, 2, TR>), dim3(total), dim3(256), 0, stream, p);
-                return hipGetLastError();
-            }
-            if (bn32) {
-                DSALT_LAUNCH("attn_fwd", (fwd_kernel<T, D, 32, 1, TR>), dim3(total), dim3(256), 0, stream, p);
-                return hipGetLastError();
-            }
-        } else if constexpr (!TR) {  // head_dim 128 (inference shapes)
-            // two row groups keep 32-key chunks (with 64-key chunks they would spill at 256 VGPRs)
-            const bool bn64 = (variant & DSALT_VARIANT_FWD_BN64) != 0;
-            const bool w8 = (variant & DSALT_VARIANT_FWD_8W) != 0 && (p.block_size == 0 || p.block_size % 128 == 0);
-            if (w8) {
-                DSALT_LAUNCH("attn_fwd", (fwd_kernel<T, D, BN, 1, TR, false, 8>),
-                             dim3(p.n_heads * p.num_seqs * ceil_div(p.n_tiles, 2)), dim3(512), 0, stream, p);
-                return hipGetLastError();
-            }
-            if (rg2) {
-                DSALT_LAUNCH("attn_fwd", (fwd_kernel<T, D, BN, 2, TR>), dim3(total), dim3(256), 0, stream, p);
-                return hipGetLastError();
-            }
-            if (bn64) {
-                DSALT_LAUNCH("attn_fwd", (fwd_kernel<T, D, 64, 1, TR>), dim3(total), dim3(256), 0, stream, p);
-                return hipGetLastError();
-            }
+    if constexpr (sizeof(T) == 2 && D == 64) {
+        if (t.rows == 128) {
+            if (t.keys == 32) DSALT_LAUNCH("attn_fwd", (fwd_kernel<T, D, 32, 2, TR>), grid, block, 0, stream, p);
+            else DSALT_LAUNCH("attn_fwd", (fwd_kernel<T, D, BN, 2, TR>), grid, block, 0, stream, p);
+            return hipGetLastError();
+        }
+        if (t.keys == 32) {
+            DSALT_LAUNCH("attn_fwd", (fwd_kernel<T, D, 32, 1, TR>), grid, block, 0, stream, p);
+            return hipGetLastError();
+        }
+    } else if constexpr (sizeof(T) == 2 && !TR) {
+        if (t.rows == 128) {
+            if (t.waves == 8) DSALT_LAUNCH("attn_fwd", (fwd_kernel<T, D, BN, 1, TR, false, 8>), grid, block, 0, stream, p);
+            else DSALT_LAUNCH("attn_fwd", (fwd_kernel<T, D, BN, 2, TR>), grid, block, 0, stream, p);
+            return hipGetLastError();
+        }
+        if (t.keys == 64) {
+            DSALT_LAUNCH("attn_fwd", (fwd_kernel<T, D, 64, 1, TR>), grid, block, 0, stream, p);
+            return hipGetLastError();
         }
     }
-    const int total = p.n_heads * p.num_seqs * p.n_tiles;
-    DSALT_LAUNCH("attn_fwd", (fwd_kernel<T, D, BN, 1, TR>), dim3(total), dim3(256), 0, stream, p);
+    DSALT_LAUNCH("attn_fwd", (fwd_kernel<T, D, BN, 1, TR>), grid, block, 0, stream, p);
     return hipGetLastError();
 }
 

@@ -276,6 +276,20 @@ size_t dsalt_plan_bytes(const dsalt_problem* p) {
     return dsalt::plan_bytes(attn_common(*p, 1.0f));
 }
 
+int dsalt_fwd_tile(const dsalt_problem* p, int32_t variant, int32_t* rows, int32_t* keys, int32_t* waves) {
+    if (!p || !rows || !keys || !waves) return fail(DSALT_ERR_INVALID, "null argument");
+    const int rc = check_problem(*p, true);
+    if (rc) return rc;
+    if (variant & ~DSALT_VARIANT_MASK) return fail(DSALT_ERR_INVALID, "unknown variant bits 0x%x", variant);
+    dsalt::AttnParams a = attn_common(*p, 1.0f);
+    a.variant = variant;
+    const dsalt::FwdTile t = dsalt::fwd_tile(a, false);
+    *rows = t.rows;
+    *keys = t.keys;
+    *waves = t.waves;
+    return DSALT_OK;
+}
+
 static int check_f32out(const dsalt_fwd_args* a, const float* out_f32) {
     if (!out_f32 || !aligned16(out_f32)) return fail(DSALT_ERR_INVALID, "out_f32 must be non-null and 16-byte aligned");
     if (a->p.dtype == DSALT_DTYPE_F32) return fail(DSALT_ERR_UNSUPPORTED, "out_f32 goes with 16-bit tensors");

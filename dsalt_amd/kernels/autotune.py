@@ -6,13 +6,16 @@ one fwd+bwd step per candidate with GPU events and caching the fastest
 choice (``dsalt_triton_bwd.py:276-277``).  The gfx950 kernels are compiled in a few tilings
 per (dtype, head_dim) -- 64 query rows per 256-thread block (4 waves x 16 rows, one query
 row per lane), key chunks of BLOCK_N rows staged in LDS, 16x16x32 MFMA tiles -- selected at
-run time by the ``variant`` bits of the C ABI (``DSALT_VARIANT_*``):
+run time by the ``variant`` bits of the C ABI (``DSALT_VARIANT_*``).  Without a forward bit the
+library picks the forward's blocks by the call's size; the bits name a tiling for every size:
 
-  * FWD_BN32  forward key chunks of 32 instead of 64 rows (16-bit, head_dim 64);
+  * FWD_BN32  forward key chunks of 32 instead of 64 rows (16-bit, head_dim 64; at head_dim 128,
+              whose chunks have 32 rows, the 64-row blocks at any size);
   * FWD_RG2   forward blocks of 128 rows, two 16-row groups per wave (16-bit; for head_dim 64
               with FWD_BN32 the kernel is held at four waves per SIMD);
   * FWD_BN64  forward key chunks of 64 instead of 32 rows (16-bit, head_dim 128, inference;
-              ignored with FWD_RG2);
+              ignored with FWD_RG2; at head_dim 64, whose chunks have 64 rows, the 64-row blocks
+              at any size);
   * FWD_8W    forward blocks of 128 rows in eight waves, one row group each: every staged key
               chunk serves twice the rows (16-bit, head_dim 128, inference; ignores FWD_RG2 and
               FWD_BN64);
@@ -48,7 +51,9 @@ def _device_key(head_dim: int, device, dtype=torch.bfloat16) -> tuple:
     return (int(head_dim), _elem_bytes(dtype), str(name))
 
 
-def _config_of(head_dim: int, elem_bytes: int, variant: int) -> dict:
+def _config_of(head_dim: int, elem_bytes: int, variant: int, tile=None) -> dict:
+    """The config of a variant; ``tile(variant)`` (a runner's ``forward_tile``) gives the forward
+    blocks a call of its size runs, else those of the compiled default are named."""
     hd = 64 if head_dim <= 64 else 128
     bn, bnq, bq = _TILES[(hd, 4 if elem_bytes == 4 else 2)]
     half = elem_bytes == 2
@@ -63,19 +68,24 @@ def _config_of(head_dim: int, elem_bytes: int, variant: int) -> dict:
         bm = 128
     if tunable and variant & VARIANT_DQ_BN64:
         bnq = 64
-    return {"BLOCK_M": bm, "BLOCK_N": bn, "BLOCK_N_BWD": bnq, "BLOCK_Q_BWD": bq, "num_warps": 8 if w8 else 4,
+    warps = 8 if w8 else 4
+    if tile is not None:
+        bm, bn, warps = tile(variant)
+    return {"BLOCK_M": bm, "BLOCK_N": bn, "BLOCK_N_BWD": bnq, "BLOCK_Q_BWD": bq, "num_warps": warps,
             "num_stages": 2, "LMK_ROWS": 512 if variant & VARIANT_LMK_SHORT else 1024, "variant": int(variant)}
 
 
 def _heuristic_config(head_dim: int, device=None, elem_bytes: int = 2) -> dict:
-    """The library's default tiling (variant 0: the compiled default tiles below; large 16-bit
-    forwards take their 128-row tiling by themselves)."""
+    """The library's default (variant 0), named by its compiled default tiles (calls of some size
+    run others: _config_of's ``tile``)."""
     return _config_of(head_dim, elem_bytes, 0)
 
 
-def _candidate_configs(head_dim: int, device=None, elem_bytes: int = 2) -> list[dict]:
+def _candidate_configs(head_dim: int, device=None, elem_bytes: int = 2, tile=None) -> list[dict]:
     """Every tiling the compiled kernels offer for the shape (the heuristic first): the forward
-    tilings with the default backward, then the backward tilings with the default forward."""
+    tilings with the default backward, then the backward tilings with the default forward.  With
+    ``tile`` (as _config_of's), each forward tiling once, the 64-row blocks among them where the
+    library's own choice is another."""
     if head_dim == 64 and elem_bytes == 2:
         variants = [0, VARIANT_FWD_BN32, VARIANT_FWD_RG2, VARIANT_FWD_RG2 | VARIANT_FWD_BN32,
                     VARIANT_DQ_BN64, VARIANT_LMK_SHORT, VARIANT_DQ_BN64 | VARIANT_LMK_SHORT]
@@ -83,7 +93,11 @@ def _candidate_configs(head_dim: int, device=None, elem_bytes: int = 2) -> list[
         variants = [0, VARIANT_FWD_RG2, VARIANT_FWD_BN64, VARIANT_FWD_8W, VARIANT_LMK_SHORT]
     else:
         variants = [0, VARIANT_LMK_SHORT]
-    return [_config_of(head_dim, elem_bytes, v) for v in variants]
+    if tile is not None and elem_bytes == 2:
+        variants.insert(1, VARIANT_FWD_BN64 if head_dim == 64 else VARIANT_FWD_BN32)
+        own = tile(0)
+        variants = [v for v in variants if v == 0 or v & _BWD_BITS or tile(v) != own]
+    return [_config_of(head_dim, elem_bytes, v, tile) for v in variants]
 
 
 # variant bits of the forward kernels and of the backward kernels (independent choices)
@@ -150,7 +164,9 @@ def autotune_blocks(head_dim: int, device, make_runner, verbose: bool = True, dt
     """Time ``make_runner(cfg)()`` (one fwd+bwd with the config's tiling; ``None`` when the
     config cannot run) for each candidate; cache and return the fastest config.  The GPU is
     warmed up on the first candidate before any timing, and the candidates are timed
-    ``rounds`` times in rotated order, each keeping its best time.  When the runners expose
+    ``rounds`` times in rotated order, each keeping its best time.  A make_runner with a
+    ``forward_tile(variant)`` (``operator_runner``'s has one) lets the configs name the blocks that
+    run at its size.  When the runners expose
     their phases (``runner.forward`` / ``runner.backward``, as ``operator_runner``'s do), the
     forward tilings are timed on the forward alone and the backward tilings on the backward
     alone, and the winner combines both choices."""
@@ -158,7 +174,8 @@ def autotune_blocks(head_dim: int, device, make_runner, verbose: bool = True, dt
     if key in _TUNED_CONFIG:
         return _TUNED_CONFIG[key]
     eb = _elem_bytes(dtype)
-    cands = _candidate_configs(head_dim, device, eb)
+    tile = getattr(make_runner, "forward_tile", None)
+    cands = _candidate_configs(head_dim, device, eb, tile)
     runners, errors = [], {}
     for cfg in cands:
         runner = make_runner(cfg)
@@ -175,12 +192,12 @@ def autotune_blocks(head_dim: int, device, make_runner, verbose: bool = True, dt
         f_best = _pick([c for c, _ in fw], f_ms)
         b_best = _pick([c for c, _ in bw], b_ms)
         v = (f_best["variant"] if f_best else 0) | (b_best["variant"] if b_best else 0)
-        best = _config_of(head_dim, eb, v)
+        best = _config_of(head_dim, eb, v, tile)
         rows = [("forward", c, f_ms.get(c["variant"]), f_best) for c, _ in fw] + \
                [("backward", c, b_ms.get(c["variant"]), b_best) for c, _ in bw if b_ms]
     else:
         ms = _timed(cands, runners, lambda r: r, rounds, errors)
-        best = _pick(cands, ms) or _heuristic_config(head_dim, device, eb)
+        best = _pick(cands, ms) or _config_of(head_dim, eb, 0, tile)
         rows = [("fwd+bwd", c, ms.get(c["variant"]), best) for c in cands]
     _TUNED_CONFIG[key] = best
     if verbose:
@@ -240,4 +257,10 @@ def operator_runner(q, k, v, w, cu_seqlens, lmk_idx, dout, *, max_seqlen=None, s
         run.forward = forward
         run.backward = backward if dout is not None else None
         return run
+
+    def forward_tile(variant):
+        return ops.forward_tile(q, k, cu_seqlens, lmk_idx, max_seqlen=max_seqlen, select_mode=mode, block_size=bs,
+                                variant=variant)
+    if q.shape[-1] in (64, 128):  # the compiled head_dims
+        make_runner.forward_tile = forward_tile
     return make_runner

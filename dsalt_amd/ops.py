@@ -254,6 +254,18 @@ def plan_buffer(T: int, S: int, max_seqlen: int, device) -> torch.Tensor:
     return torch.empty(max(_lib.load().dsalt_plan_bytes(ctypes.byref(prob)), 1), dtype=torch.uint8, device=device)
 
 
+def forward_tile(q: torch.Tensor, k: torch.Tensor, cu_seqlens: torch.Tensor, lmk_idx: torch.Tensor, *, max_seqlen=None,
+                 select_mode=SELECT_GLOBAL, block_size=512, variant=VARIANT_DEFAULT):
+    """(query rows, keys a chunk, waves) of the blocks attention_forward runs for these shapes."""
+    T, H, D = q.shape
+    maxlen = max_seqlen if max_seqlen is not None else _max_seqlen(cu_seqlens)
+    prob = _problem(T, cu_seqlens.shape[0] - 1, maxlen, H, k.shape[1], D, lmk_idx.shape[-1], select_mode, block_size,
+                    dtype_code(q.dtype))
+    tile = [ctypes.c_int32() for _ in range(3)]
+    _lib.check("dsalt_fwd_tile", _lib.load().dsalt_fwd_tile(ctypes.byref(prob), int(variant), *map(ctypes.byref, tile)))
+    return tuple(t.value for t in tile)
+
+
 def _check_plan(plan, a) -> int:
     if plan is None:
         return 0

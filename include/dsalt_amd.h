@@ -353,7 +353,9 @@ int    dsalt_sort_landmarks(const dsalt_sort_args* a, dsalt_stream_t stream);
 
 /* Tile variants of the attention kernels (dsalt_fwd_args.variant, dsalt_bwd_args.variant).
  * Bits are independent; a bit a shape cannot use is ignored.  Without forward bits the
- * forward picks its tiling by the call's size (attn_fwd.hip::fwd_variant). */
+ * forward picks its tiling by the call's size (dsalt_fwd_tile tells which); the bit of a
+ * head_dim's own chunk length (FWD_BN64 at 64, FWD_BN32 at 128) names its 64-row blocks
+ * at any size. */
 #define DSALT_VARIANT_DEFAULT    0
 #define DSALT_VARIANT_FWD_BN32   1  /* forward: 32-key chunks (16-bit types, head_dim 64)        */
 #define DSALT_VARIANT_FWD_RG2    2  /* forward: two 16-row groups per wave (16-bit types)       */
@@ -365,6 +367,10 @@ int    dsalt_sort_landmarks(const dsalt_sort_args* a, dsalt_stream_t stream);
                                        each (16-bit, head_dim 128, inference operator; ignores
                                        FWD_RG2 and FWD_BN64)                                     */
 #define DSALT_VARIANT_MASK       63
+
+/* The tiling dsalt_fwd runs for the problem and variant bits: query rows, keys a chunk and
+ * waves of a block. */
+int dsalt_fwd_tile(const dsalt_problem* p, int32_t variant, int32_t* rows, int32_t* keys, int32_t* waves);
 
 /* Bytes of the row-plan buffer of dsalt_fwd_args.plan / dsalt_bwd_args.plan. */
 size_t dsalt_plan_bytes(const dsalt_problem* p);
