@@ -728,14 +728,17 @@ __global__ __launch_bounds__(64 * NW, ((sizeof(T) == 2 && D == 64 && RG == 2 && 
 //     0.93-0.99x, 8192 0.91-0.99x, 32768 0.89-0.92x (16 heads x 32768, windows up to 512: 157.4 ->
 //     146.1 us).  Short sequences leave half of a block without rows: 512 to 700 tokens 0.96-1.02x,
 //     150 to 320 1.05-1.11x, 64 1.22x;
-//   head_dim 128: FWD_8W from kW8Tiles on, where staging the key chunks bounds the kernel: 32768
-//     tiles 0.945-0.997x (16 heads x 131072, 256 landmarks: 1130 -> 1077 us); 8192 tiles
-//     0.93-1.12x and 2048 0.96-1.07x (slower for windows below 512), so these keep four waves.
+//   head_dim 128: FWD_8W from kW8Tiles on where every head has its own keys and sequences hold kW8Len
+//     tokens on average, so that staging the key chunks bounds the kernel: 32768 tiles, windows up
+//     to 256 or 512 0.92-0.99x (16 heads x 131072, windows up to 512, 256 landmarks: 1225 -> 1159 us),
+//     windows up to 64 0.97-1.03x; 24576 tiles 0.94-1.03x, 16384 0.95-1.08x.  Grouped heads find
+//     their chunks in L2 (0.93-1.11x, 1.02x on average), and shorter sequences fill fewer of the
+//     128 rows (8192 tokens up to 1.04x, 512 1.12x, 64 1.23x).
 // The training variant keeps 64-row blocks: its two row groups are held to too few registers
 // (1.13-1.26x from 1536 tiles on).
 // Sets of more than kSetSlots landmarks, and block-causal sets of a block_size that is not a
 // multiple of 64, take the default tiling's wide instantiation (variant bits ignored).
-constexpr int64_t kRg2Tiles = 6144, kRg2Len = 1024, kW8Tiles = 16384;
+constexpr int64_t kRg2Tiles = 6144, kRg2Len = 1024, kW8Tiles = 32768, kW8Len = 65536;
 
 FwdTile fwd_tile(const AttnParams& p, bool train) {
     const bool half = p.dtype != DSALT_DTYPE_F32;
@@ -751,7 +754,8 @@ FwdTile fwd_tile(const AttnParams& p, bool train) {
         if (whole && (rg2 || (!chosen && by_size))) t.rows = 128;
         if (bn32) t.keys = 32;
     } else if (!train) {
-        if (whole && (w8 || (!chosen && tiles >= kW8Tiles))) {
+        const bool by_size = tiles >= kW8Tiles && p.n_kv_heads == p.n_heads && p.total_len >= kW8Len * p.num_seqs;
+        if (whole && (w8 || (!chosen && by_size))) {
             t.rows = 128;
             t.waves = 8;
         } else if (whole && rg2) {

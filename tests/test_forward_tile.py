@@ -29,6 +29,14 @@ def _tile(T, H, D, variant=0, S=1, G=None, K=64, block=0, dt=_lib.DTYPE_BF16):
     (dict(T=24576, H=16, D=64, K=513), (64, 64, 4)),
     (dict(T=24576, H=16, D=64, dt=_lib.DTYPE_F32), (64, 32, 4)),
     (dict(T=100, H=4, D=128), (64, 32, 4)),
+    (dict(T=131071, H=16, D=128), (64, 32, 4)),                    # one token under 32768 tiles
+    (dict(T=131072, H=16, D=128), (128, 32, 8)),
+    (dict(T=131072, H=16, D=128, block=512), (128, 32, 8)),
+    (dict(T=131072, H=16, D=128, block=64), (64, 32, 4)),
+    (dict(T=131072, H=16, D=128, S=2), (128, 32, 8)),              # 65536 tokens a sequence
+    (dict(T=131072, H=16, D=128, S=3), (64, 32, 4)),
+    (dict(T=131072, H=16, D=128, G=8), (64, 32, 4)),               # grouped heads
+    (dict(T=65536, H=64, D=128, S=1024), (64, 32, 4)),             # many short sequences
     (dict(T=100, H=4, D=128, dt=_lib.DTYPE_F32), (64, 16, 4)),
 ])
 def test_tile_by_size(args, want):

@@ -18,7 +18,7 @@ DEV = "cuda"
     ([20001, 6000], 16, 8, 64, torch.float16, 0, False),
     ([24600], 16, 16, 64, torch.bfloat16, 256, False),
     ([65, 400, 64] * 48, 16, 16, 64, torch.bfloat16, 0, False),  # short sequences
-    ([8321], 128, 128, 128, torch.bfloat16, 0, False),
+    ([65601], 32, 32, 128, torch.bfloat16, 0, False),     # eight waves, an odd number of tiles
     ([8200], 16, 16, 64, torch.bfloat16, 0, True),
     ([24600], 16, 8, 64, torch.float16, 0, True),
 ])
