@@ -174,11 +174,9 @@ class DSALTAttention(nn.Module):
 
     def _selectors(self, x):
         """(integer windows [T] int32, alpha [H] float32) of the inference branch: one kernel after
-        the gate's product, or the torch expressions where a subclass redefines them or the tensors'
-        types differ (autocast)."""
-        cls = type(self)
-        if cls._window_sizes is DSALTAttention._window_sizes and cls._alpha is DSALTAttention._alpha \
-                and cls._window_continuous is DSALTAttention._window_continuous and x.is_cuda:
+        the gate's product, or the torch expressions where the methods are replaced (by a subclass,
+        on the class or on the instance) or the tensors' types differ (autocast)."""
+        if x.is_cuda and all(getattr(getattr(self, n), "__func__", None) is f for n, f in _OWN_SELECTORS.items()):
             gate = self.win_gate(x)
             if gate.dtype == self.alpha_w.dtype and gate.dim() == 2 and gate.shape[1] == 1 \
                     and gate.dtype in (torch.float32, torch.bfloat16, torch.float16):
@@ -266,3 +264,7 @@ class DSALTAttention(nn.Module):
                               cu_list=cu_list, block_size=self.block_size)
         self._last_P = None
         return self._apply_out_proj(out.view(total_len, self.d_model)), self._aux_zero(x.device, x.dtype)
+
+
+# what the selector kernel computes; anything else in their place is called instead
+_OWN_SELECTORS = {n: DSALTAttention.__dict__[n] for n in ("_alpha", "_window_continuous", "_window_sizes")}

@@ -1,0 +1,54 @@
+"""Which windows and score weights the attention layer runs at inference: its own methods' values,
+also where a program replaces them, and one evaluation of the window gate a call."""
+from __future__ import annotations
+
+import types
+
+import pytest
+import torch
+
+from dsalt_amd.modules import DSALTAttention
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _layer(dt=torch.bfloat16, **kw):
+    torch.manual_seed(2)
+    args = dict(d_model=256, n_heads=4, n_min=8, n_max=90, k_lmk=11, max_seq_len=512, n_kv_heads=2)
+    args.update(kw)
+    return DSALTAttention(**args).to(DEV, dt).eval()
+
+
+def _run(m, T=300):
+    x = torch.randn(T, 256, generator=torch.Generator(device=DEV).manual_seed(T), device=DEV).to(m.out_proj.weight.dtype)
+    with torch.no_grad():
+        return m(x, cu_seqlens=torch.tensor([0, T], dtype=torch.int32, device=DEV), cu_list=[0, T])[0]
+
+
+@pytest.mark.parametrize("where", ["instance", "class", "subclass"])
+@pytest.mark.parametrize("name", ["_alpha", "_window_continuous", "_window_sizes"])
+def test_replaced_methods_are_called(name, where, monkeypatch):
+    calls = []
+    body = {"_alpha": lambda self: torch.full((4,), 0.9, device=DEV),
+            "_window_continuous": lambda self, x: torch.full((x.shape[0],), 31.5, device=DEV),
+            "_window_sizes": lambda self, x, floor: torch.full((x.shape[0],), 17.0, device=DEV)}[name]
+
+    def repl(self, *a, **kw):
+        calls.append(name)
+        return body(self, *a, **kw)
+
+    m = _layer()
+    if where == "instance":
+        setattr(m, name, types.MethodType(repl, m))
+    elif where == "class":
+        monkeypatch.setattr(DSALTAttention, name, repl)
+    else:
+        m.__class__ = type("Own", (DSALTAttention,), {name: repl})
+    w, alpha = m._selectors(torch.randn(300, 256, device=DEV, dtype=torch.bfloat16))
+    assert calls and w.dtype == torch.int32 and alpha.dtype == torch.float32
+    if name == "_alpha":
+        assert torch.equal(alpha, torch.full_like(alpha, 0.9))
+    else:
+        assert torch.equal(w, torch.full_like(w, 31 if name == "_window_continuous" else 17))
+    assert torch.isfinite(_run(m)).all()
