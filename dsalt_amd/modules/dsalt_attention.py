@@ -87,8 +87,11 @@ class DSALTAttention(nn.Module):
     def _alpha(self) -> torch.Tensor:
         return torch.sigmoid(self.alpha_w)
 
+    def _windows_of(self, gate: torch.Tensor) -> torch.Tensor:
+        return self.n_min + torch.sigmoid(gate.squeeze(-1)) * (self.n_max - self.n_min)
+
     def _window_continuous(self, x: torch.Tensor) -> torch.Tensor:
-        return self.n_min + torch.sigmoid(self.win_gate(x).squeeze(-1)) * (self.n_max - self.n_min)
+        return self._windows_of(self.win_gate(x))
 
     @torch.no_grad()
     def _window_sizes(self, x: torch.Tensor, floor: bool) -> torch.Tensor:
@@ -181,6 +184,7 @@ class DSALTAttention(nn.Module):
             if gate.dtype == self.alpha_w.dtype and gate.dim() == 2 and gate.shape[1] == 1 \
                     and gate.dtype in (torch.float32, torch.bfloat16, torch.float16):
                 return ops.layer_selectors(gate.detach().view(-1), self.alpha_w.detach(), self.n_min, self.n_max)
+            return self._windows_of(gate).floor().clamp(min=1).to(torch.int32), self._alpha().float()
         return self._window_sizes(x, floor=True).to(torch.int32), self._alpha().float()
 
     @torch.no_grad()

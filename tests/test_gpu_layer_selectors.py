@@ -52,3 +52,21 @@ def test_replaced_methods_are_called(name, where, monkeypatch):
     else:
         assert torch.equal(w, torch.full_like(w, 31 if name == "_window_continuous" else 17))
     assert torch.isfinite(_run(m)).all()
+
+
+@pytest.mark.parametrize("alpha_dt", [torch.bfloat16, torch.float32])
+def test_the_window_gate_runs_once(alpha_dt):
+    """Also where the types differ (16-bit weights with float32 score weights): its hooks see one call."""
+    m = _layer()
+    m.alpha_w.data = m.alpha_w.data.to(alpha_dt)
+    calls = []
+    m.win_gate.register_forward_hook(lambda mod, a, y: calls.append(y))
+    x = torch.randn(300, 256, device=DEV, dtype=torch.bfloat16)
+    with torch.no_grad():
+        w, alpha = m._selectors(x)
+        assert len(calls) == 1
+        gate = calls[0].squeeze(-1)
+        ref = (m.n_min + torch.sigmoid(gate) * (m.n_max - m.n_min)).floor().clamp(min=1).int()
+    assert torch.equal(w, ref) and torch.equal(alpha, torch.sigmoid(m.alpha_w.data).float())
+    _run(m)
+    assert len(calls) == 2
