@@ -41,7 +41,7 @@ from .. import ops
 from ..kernels.dsalt_attn import dsalt_attention, pad_head_dim, padded_head_dim
 from ..kernels.dsalt_train import dsalt_train_attention
 from ..kernels.landmark_tokens_ker import hybrid_scores_per_head
-from ..kernels.selectors import _SCOPES, _compute_landmark_indices
+from ..kernels.selectors import _MODES, _SCOPES, _compute_landmark_indices
 from ..kernels.window_utils import apply_rotary_emb, build_rope_cache
 
 
@@ -203,7 +203,7 @@ class DSALTAttention(nn.Module):
             cu1 = torch.tensor([0, total_len], dtype=torch.int32, device=device)
             ops.rope_qk_(q, k, cu1, rope_cs[0].float(), rope_cs[1].float(), max_seqlen=total_len)
         w32, alpha = self._selectors(x)
-        mode = ops.SELECT_BLOCK if self.select_mode == "block" else ops.SELECT_GLOBAL
+        mode = _MODES[self.select_mode]
         # landmarks on x W_V^T without the bias, whatever the projection's; the selection's first
         # launch also writes the attention's row plan
         plan = ops.plan_buffer(total_len, cu_seqlens.shape[0] - 1, maxlen, x.device)

@@ -70,3 +70,9 @@ def test_the_window_gate_runs_once(alpha_dt):
     assert torch.equal(w, ref) and torch.equal(alpha, torch.sigmoid(m.alpha_w.data).float())
     _run(m)
     assert len(calls) == 2
+
+
+@pytest.mark.parametrize("kw", [dict(select_mode="causal"), dict(stats_scope="batch")])
+def test_unknown_modes_are_refused(kw):
+    with pytest.raises(KeyError):
+        _run(_layer(**kw))
