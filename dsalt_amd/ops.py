@@ -10,6 +10,7 @@ import ctypes
 import math
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _lib
 from ._lib import (DTYPE_BF16, DTYPE_F16, DTYPE_F32, SELECT_BLOCK, SELECT_GLOBAL, STATS_PACKED,
@@ -677,13 +678,30 @@ def layer_selectors(gate: torch.Tensor, alpha_w: torch.Tensor, n_min, n_max):
     return w, alpha
 
 
+def _plain(*ts) -> bool:
+    """Whether the tensors are ordinary ones outside every transform, trace and dispatch mode, so that a
+    kernel may read their memory where the torch operations in its place would be seen by it."""
+    if torch.jit.is_tracing() or torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack():
+        return False
+    for t in ts:
+        if t is None:
+            continue
+        if type(t) not in (torch.Tensor, torch.nn.Parameter) or torch._C._functorch.is_functorch_wrapped_tensor(t):
+            return False
+        if forward_ad._current_level >= 0 and t.is_floating_point() and forward_ad.unpack_dual(t).tangent is not None:
+            return False
+    return True
+
+
 def sort_landmarks(idx: torch.Tensor, bias: torch.Tensor | None = None):
     """Sort each set ascending with -1 last (the order the kernels require); returns
-    (sorted int32 indices, bias permuted the same way or None, permutation)."""
-    b_ok = bias is None or (bias.element_size() in (2, 4) and bias.device == idx.device and bias.shape == idx.shape
-                            and not (torch.is_grad_enabled() and bias.requires_grad))
-    if idx.device.type == "cuda" and idx.dtype in (torch.int32, torch.int64) and b_ok \
-            and 0 < idx.shape[-1] <= MAX_LANDMARKS and idx.numel():
+    (sorted int32 indices, bias permuted the same way or None, permutation).  One kernel for ordinary
+    tensors; differentiable, batched and traced ones go through the torch operations."""
+    if idx.is_cuda and _plain(idx, bias) and idx.dtype in (torch.int32, torch.int64) and idx.dim() > 0 \
+            and 0 < idx.shape[-1] <= MAX_LANDMARKS and idx.numel() \
+            and (bias is None or (bias.element_size() in (2, 4) and bias.device == idx.device
+                                  and bias.shape == idx.shape
+                                  and not (torch.is_grad_enabled() and bias.requires_grad))):
         src = idx.detach().contiguous()
         out = torch.empty(src.shape, dtype=torch.int32, device=src.device)
         perm = torch.empty(src.shape, dtype=torch.int64, device=src.device)

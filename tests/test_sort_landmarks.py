@@ -86,6 +86,31 @@ def test_sort_landmarks(K, kind, dt, bdt):
 
 
 @pytest.mark.gpu
+def test_sort_landmarks_under_transforms():
+    """Forward-mode tangents, vmap and traces see the torch operations; so does a 0-dim set."""
+    from torch.autograd import forward_ad as fw
+    from torch.fx.experimental.proxy_tensor import make_fx
+    g = torch.Generator().manual_seed(5)
+    idx = torch.stack([torch.randperm(500, generator=g)[:9] for _ in range(12)]).view(3, 4, 1, 9).to(DEV)
+    idx[0, :, 0, 3] = -1
+    bias, tan = (torch.randn(idx.shape, generator=g).to(DEV) for _ in range(2))
+    ro, rb, rp = ops.sort_landmarks(idx, bias)
+    with fw.dual_level():
+        o, b, p = ops.sort_landmarks(idx, fw.make_dual(bias, tan))
+        assert torch.equal(o, ro) and torch.equal(fw.unpack_dual(b).tangent, tan.gather(-1, rp))
+    _, t = torch.func.jvp(lambda x: ops.sort_landmarks(idx, x)[1], (bias,), (tan,))
+    assert torch.equal(t, tan.gather(-1, rp))
+    for a, r in zip(torch.vmap(ops.sort_landmarks)(idx, bias), (ro, rb, rp)):
+        assert torch.equal(a, r)
+    other, obias = idx.flip(-1), bias * 2
+    want = ops.sort_landmarks(other, obias)
+    for f in (make_fx(ops.sort_landmarks)(idx, bias), torch.jit.trace(ops.sort_landmarks, (idx, bias), check_trace=False)):
+        for a, r in zip(f(other, obias), want):
+            assert torch.equal(a, r)
+    assert int(ops.sort_landmarks(torch.tensor(7, device=DEV))[0]) == 7
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("H,G,D,dt,T", [(4, 4, 64, torch.bfloat16, 1601), (4, 2, 64, torch.float16, 130),
                                         (16, 4, 64, torch.bfloat16, 6500), (4, 2, 128, torch.bfloat16, 777)])
 @pytest.mark.parametrize("train", [False, True])
