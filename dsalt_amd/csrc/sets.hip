@@ -3,11 +3,12 @@
 //
 // One block per set.  Sets a selection made are already in order: the block compares
 // neighbours and copies.  Else each slot counts the slots that come before it (equal
-// positions keep their order), k^2 / threads LDS reads: the sets are small (k <= 2048, usually
-// at most 128), so one launch is bound by its latency, where a general radix sort with the
-// selects, conversions and gathers around it took eleven launches (8 sets of 64 slots: 21.7 of
-// about 45 us on the GPU in the sort alone, with their host time more than the attention
-// forward beside them).
+// positions keep their order), k^2 / threads LDS reads: the sets are small (usually at most 128
+// slots), so one launch is bound by its latency, where a general radix sort with the selects,
+// conversions and gathers around it took eleven launches (8 sets of 64 slots: 21.7 of about 45 us
+// on the GPU in the sort alone, with their host time more than the attention forward beside
+// them).  From about 512 slots on the count is the slower way for sets out of order (8 sets of
+// 1024: 214 us against 57), and a caller with such sets sorts them otherwise.
 #include "sets.h"
 
 #include "common.h"

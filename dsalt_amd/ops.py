@@ -693,12 +693,19 @@ def _plain(*ts) -> bool:
     return True
 
 
+# largest set the kernel orders: it counts k^2 comparisons of a set out of order.  Call with biases, us,
+# kernel / torch sort: 8 shuffled sets of 256 slots 16 / 56, of 512 56 / 57, of 1024 214 / 57, of 2048
+# 854 / 57; 4096 sets of 256 51 / 151, of 512 178 / 171, of 1024 689 / 231 (sets in order at any k: 12)
+_SORT_SLOTS = 512
+
+
 def sort_landmarks(idx: torch.Tensor, bias: torch.Tensor | None = None):
     """Sort each set ascending with -1 last (the order the kernels require); returns
     (sorted int32 indices, bias permuted the same way or None, permutation).  One kernel for ordinary
-    tensors; differentiable, batched and traced ones go through the torch operations."""
+    tensors of up to _SORT_SLOTS slots a set; larger sets and differentiable, batched and traced
+    tensors go through the torch operations."""
     if idx.is_cuda and _plain(idx, bias) and idx.dtype in (torch.int32, torch.int64) and idx.dim() > 0 \
-            and 0 < idx.shape[-1] <= MAX_LANDMARKS and idx.numel() \
+            and 0 < idx.shape[-1] <= _SORT_SLOTS and idx.numel() \
             and (bias is None or (bias.element_size() in (2, 4) and bias.device == idx.device
                                   and bias.shape == idx.shape
                                   and not (torch.is_grad_enabled() and bias.requires_grad))):
@@ -719,7 +726,7 @@ def sort_landmarks(idx: torch.Tensor, bias: torch.Tensor | None = None):
         return out, b, perm
     big = torch.iinfo(torch.int32).max
     key = torch.where(idx < 0, torch.full_like(idx, big), idx).to(torch.int64)
-    srt, perm = key.sort(dim=-1)
+    srt, perm = key.sort(dim=-1, stable=True)
     out = torch.where(srt == big, torch.full_like(srt, -1), srt).to(torch.int32)
     b = bias.gather(-1, perm) if bias is not None else None
     return out, b, perm

@@ -86,6 +86,22 @@ def test_sort_landmarks(K, kind, dt, bdt):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("K,kernel", [(1, True), (512, True), (513, False), (2048, False)])
+def test_large_sets_are_not_counted(K, kernel, monkeypatch):
+    """Sets past the kernel's size, which it would order in k^2 steps, go to the library sort."""
+    called, check = [], _lib.check
+    monkeypatch.setattr(_lib, "check", lambda name, rc: (called.append(name), check(name, rc)))
+    idx = torch.randint(0, 7, (3, 1, 1, K), generator=torch.Generator().manual_seed(K))
+    out, _, perm = ops.sort_landmarks(idx.to(DEV))
+    ro, _, rp = _reference(idx, None)
+    assert torch.equal(out.cpu(), ro) and torch.equal(perm.cpu(), rp)
+    assert called == (["dsalt_sort_landmarks"] if kernel else [])
+    monkeypatch.setattr(ops, "_SORT_SLOTS", 2048)  # the kernel itself takes them all
+    out, _, perm = ops.sort_landmarks(idx.to(DEV))
+    assert called and torch.equal(out.cpu(), ro) and torch.equal(perm.cpu(), rp)
+
+
+@pytest.mark.gpu
 def test_sort_landmarks_under_transforms():
     """Forward-mode tangents, vmap and traces see the torch operations; so does a 0-dim set."""
     from torch.autograd import forward_ad as fw
