@@ -20,7 +20,12 @@
 // compares its index with the target in 64 bits (4001 rows: 688 -> 655 us; 32000 columns 145 ->
 // 115).  Three blocks per CU, held by their LDS request, keep the rows in flight within the
 // memory-side cache for the second read (655 -> 630 us; four blocks 655, two 644): 3.9 TB/s of one
-// read and one write, 5.8 counting the second read.
+// read and one write, 5.8 counting the second read.  They are asked for only where there is a second
+// pass bound by memory, over rows of at least kCeLdsRow bytes (4001 rows, three blocks / four, us:
+// 16-bit 16384 columns 57 / 60, 32000 111 / 113, 128256 528 / 544; float32 32000 258 / 262, 128256
+// 1156 / 1193).  Elsewhere four blocks hide more: 16-bit 1003 columns 30 / 26, 4096 34 / 29; float32
+// 1003 35 / 30; 128256 columns without gradients 197 / 186, softcap 909 / 860, class weights
+// 2055 / 1955.
 #include "ce.h"
 #include "common.h"
 #include "timing.h"
@@ -30,7 +35,8 @@ namespace dsalt {
 namespace {
 
 constexpr int kCeThreads = 512;
-constexpr int kCeLds = 50000;  // dynamic LDS requested (unused): three blocks per CU
+// dynamic LDS requested (unused) for three blocks per CU, and the smallest row it is requested for
+constexpr int kCeLds = 50000, kCeLdsRow = 32768;
 
 struct RowStats {
     float m, d, sx;  // running max, sum of exp(x - m), label-smoothing sum
@@ -234,15 +240,17 @@ hipError_t ce_launch(const CeParams& p, hipStream_t stream) {
     if (p.rows == 0) return hipSuccess;
     const dim3 grid((unsigned)p.rows);
     const bool plain = p.ce_weight == nullptr && !(p.softcap > 0.f);
+    const int64_t row_bytes = (int64_t)p.n_cols * (p.dtype == 0 ? 4 : 2);
+    const unsigned lds = plain && p.grads && row_bytes >= kCeLdsRow ? kCeLds : 0;
     switch (p.dtype) {
-        case 0: DSALT_LAUNCH("ce_rows", (ce_kernel<float, false>), grid, dim3(kCeThreads), kCeLds, stream, p); break;
+        case 0: DSALT_LAUNCH("ce_rows", (ce_kernel<float, false>), grid, dim3(kCeThreads), lds, stream, p); break;
         case 1:
-            if (plain) DSALT_LAUNCH("ce_rows", (ce_kernel<bf16, true>), grid, dim3(kCeThreads), kCeLds, stream, p);
-            else DSALT_LAUNCH("ce_rows", (ce_kernel<bf16, false>), grid, dim3(kCeThreads), kCeLds, stream, p);
+            if (plain) DSALT_LAUNCH("ce_rows", (ce_kernel<bf16, true>), grid, dim3(kCeThreads), lds, stream, p);
+            else DSALT_LAUNCH("ce_rows", (ce_kernel<bf16, false>), grid, dim3(kCeThreads), lds, stream, p);
             break;
         default:
-            if (plain) DSALT_LAUNCH("ce_rows", (ce_kernel<f16, true>), grid, dim3(kCeThreads), kCeLds, stream, p);
-            else DSALT_LAUNCH("ce_rows", (ce_kernel<f16, false>), grid, dim3(kCeThreads), kCeLds, stream, p);
+            if (plain) DSALT_LAUNCH("ce_rows", (ce_kernel<f16, true>), grid, dim3(kCeThreads), lds, stream, p);
+            else DSALT_LAUNCH("ce_rows", (ce_kernel<f16, false>), grid, dim3(kCeThreads), lds, stream, p);
             break;
     }
     return hipGetLastError();
