@@ -98,9 +98,10 @@ __device__ __forceinline__ void edge_terms(const AttnParams& p, float wt, int d,
 // keys from the unclamped window start lo_u = i - floor(wt): key lo_u + k sits at
 // wt - d = frac(wt) + k.  For win_edge <= 4 the kernels read a row's edge terms from an LDS
 // table built once per row (no transcendentals per key): entry k at offset k, zeros after
-// them (the core), and kEdgeLead zeros before a wave's 16 rows (before a later row of the wave
+// them (the core), and kEdgeLead floats before a wave's 16 rows (before a later row of the wave
 // lie the zeros of the one before it), so the four keys of a lane from any offset, clamped to
-// [-4, 4], read the right entries where the mask lets them count and zeros elsewhere.  Four-way
+// [-4, 4], read the right entries where the mask lets them count and others elsewhere (keys
+// before the window start: never selected by the mask).  Four-way
 // selects from registers instead cost 32 VALU instructions per subtile and term, more than
 // the rest of its scores, and the registers of two row groups spilled.
 constexpr int kEdgeTab = 4;
@@ -108,13 +109,15 @@ constexpr int kEdgeRow = 8, kEdgeLead = 4;
 constexpr int kEdgeWave = kEdgeLead + 16 * kEdgeRow;  // floats of a wave's table
 // offset of the row of accumulator lane `lane` in the table of wave slot `slot`
 __device__ __forceinline__ int edge_row(int slot, int lane) { return slot * kEdgeWave + kEdgeLead + (lane & 15) * kEdgeRow; }
-// writes the row's entries, one per 16-lane group (every lane of the wave calls it); grad: null
-// or a second table of d bias / d wt.  Read by the same wave only.
+// writes the row's entries, one per 16-lane group (every lane of the wave calls it), and with LEAD
+// the floats before the wave's rows; grad: null or a second table of d bias / d wt.  Read by the
+// same wave only.
+template <bool LEAD>
 __device__ __forceinline__ void edge_table(const AttnParams& p, float wt, int lane, int row, float* bias, float* grad) {
     const int g = lane >> 4;
     float b, d;
     edge_terms(p, wt - floorf(wt) + (float)g, 0, b, d);
-    const bool lead = (lane & 15) == 0;
+    const bool lead = LEAD && (lane & 15) == 0;
     bias[row + g] = b;
     bias[row + 4 + g] = 0.f;
     if (lead) bias[row - kEdgeLead + g] = 0.f;

@@ -76,6 +76,14 @@ __device__ __forceinline__ int load_set(const AttnParams& p, int64_t set_off, in
 }
 
 // -------------------------------------------------------------------- dQ
+template <typename T, int ELEMS, int LCAP>
+struct DqShared {
+    __attribute__((aligned(16))) T Ks[2][ELEMS];
+    __attribute__((aligned(16))) T Vs[2][ELEMS];
+    __attribute__((aligned(16))) int lpos[LCAP];
+    __attribute__((aligned(16))) float lbs[LCAP];
+};
+
 // TR: training variant -- band keys near the window start carry the soft edge bias,
 // and the lane also sums dS * d(bias)/d(w~) of its row into dw_h.
 // LK: sets of more than kSetSlots landmarks (inference operator), staged by a loop.
@@ -86,11 +94,19 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 && D == 64) ? (BN == 32 ? (TR 
     constexpr bool kHalf = sizeof(T) == 2;
     constexpr int LCAP = LK ? kMaxLandmarks : kSetSlots;
     typedef Tile<T, D, BN, 256, (BN == 64 ? 8 : Pad<T, D>::R)> KT;
-    __shared__ __attribute__((aligned(16))) T Ks[2][KT::ELEMS];
-    __shared__ __attribute__((aligned(16))) T Vs[2][KT::ELEMS];
-    __shared__ int lpos[LCAP];
-    __shared__ __attribute__((aligned(16))) float lbs[LCAP];
-    __shared__ float etb[TR ? 4 * kEdgeWave : 1], etg[TR ? 4 * kEdgeWave : 1];
+    __shared__ DqShared<T, KT::ELEMS, LCAP> sm;
+    auto &Ks = sm.Ks, &Vs = sm.Vs;
+    int* const lpos = sm.lpos;
+    float* const lbs = sm.lbs;
+    // training variant: the band's soft-edge tables over the landmark slots, which it no longer reads
+    // (beside them the 64-key blocks lost a wave per SIMD: 8 heads, 4 x 8192, 100 us against 85): bias
+    // and gradient of wave w's rows at 256 w and 256 w + 128.  Before a gradient table lie zeros of
+    // its own wave, before a bias table what no mask selects; before the first, the padding of the
+    // last V row.
+    constexpr int kEdgeTable = 16 * kEdgeRow;
+    float* const etb = (float*)sm.lpos;
+    static_assert(!TR || 8 * kEdgeTable <= 2 * LCAP, "the soft-edge tables do not fit the landmark slots");
+    static_assert(!TR || (KT::RS - D) * sizeof(T) >= sizeof(float) * kEdgeLead, "no padding before the soft-edge tables");
     // block scalars live in the second K buffer until the first chunk is staged there
     int* red = (int*)Ks[1];
 
@@ -202,9 +218,7 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 && D == 64) ? (BN == 32 ? (TR 
         cnt = lower_bound_i(lpos, nvalid, lo);
         if (TR) wt = wt_raw;
     }
-    // soft-edge bias and window gradient of keys lou .. lou+3 (training variant, win_edge <= 4)
-    const int eo = edge_row(uw, lane);
-    if (TR && p.edge_keys <= kEdgeTab) edge_table(p, wt, lane, eo, etb, etg);
+    const int eo = uw * 2 * kEdgeTable + (lane & 15) * kEdgeRow;  // the row's soft-edge entries
     const int lo_edge = TR ? wLmax + p.edge_keys : wLmax;  // keys from here on carry no edge bias
     float dwacc = 0.f;
     // per-row data of the key-parallel passes, head-major: a head's rows are contiguous
@@ -350,12 +364,12 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 && D == 64) ? (BN == 32 ? (TR 
                     for (int r = 0; r < 4; ++r) ci[r] = (unsigned)(x0 + r) <= wd ? 0.f : NEG;
                     if (TR && a < lo_edge) {
                         if (p.edge_keys <= kEdgeTab) {
-                            // (a masked key's dS is 0, so its gradient entry counts for nothing)
+                            // (a masked key's dS is 0, so its gradient entry, a finite one, counts for nothing)
                             const int at = edge_at(eo, a + lane_off - lou);
 #pragma unroll
                             for (int r = 0; r < 4; ++r) {
                                 ci[r] = (unsigned)(x0 + r) <= wd ? etb[at + r] : NEG;
-                                eg[r] = etg[at + r];
+                                eg[r] = etb[kEdgeTable + at + r];
                             }
                         } else {
 #pragma unroll
@@ -405,6 +419,7 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 && D == 64) ? (BN == 32 ? (TR 
         __syncthreads();
     };
     for (int n = 0; n < nlmk; ++n) process(n, std::false_type{});
+    if (TR && p.edge_keys <= kEdgeTab) edge_table<false>(p, wt, lane, eo, etb, etb + kEdgeTable);
     for (int n = nlmk; n < nchunks; ++n) process(n, std::true_type{});
     if (TR) {
         const float dw = sum_g4(dwacc);

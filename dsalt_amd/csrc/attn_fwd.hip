@@ -679,7 +679,7 @@ __global__ __launch_bounds__(64 * NW, ((sizeof(T) == 2 && D == 64 && RG == 2 && 
 #pragma unroll
         for (int u = 0; u < RG; ++u) {
             rg[u].eo = edge_row(u * NW + uw, lane);
-            edge_table(p, rg[u].wt, lane, rg[u].eo, etab, nullptr);
+            edge_table<true>(p, rg[u].wt, lane, rg[u].eo, etab, nullptr);
         }
     }
     for (int n = nlmk; n < nchunks; ++n) process(n, std::true_type{});
