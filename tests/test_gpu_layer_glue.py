@@ -90,7 +90,9 @@ def test_layer_without_its_selector_kernel_is_the_same(dt):
 def test_lm_loss_layouts(rows, V, bias, dt, accum, monkeypatch):
     """Loss and gradients against plain torch in float32 on the 16-bit logits the loss is defined
     on.  The gradient of a logit is rounded to the type once, the sums once more, a second chunk once
-    more: relative 2-norm at most 4 u (u = 2^-9, 2^-12), float32 1e-5."""
+    more: relative 2-norm at most 3 u (u = 2^-8, 2^-11); asked for is 2 u in bfloat16, where every
+    rounding at its largest would be needed for more, 4 u in float16 (gradients of 1e-6 reach its
+    subnormals), and 1e-5 in float32."""
     g = torch.Generator(device=DEV).manual_seed(rows + V)
     H = 96
     x = torch.randn(rows, H, generator=g, device=DEV).to(dt).requires_grad_(True)
@@ -108,7 +110,7 @@ def test_lm_loss_layouts(rows, V, bias, dt, accum, monkeypatch):
     d[~keep] = 0
     d = (d / n).to(dt).float()
     ref = [d @ w.detach().float(), d.T @ x.detach().float()] + ([d.sum(0)] if bias else [])
-    tol = {torch.bfloat16: 4 * 2.0 ** -9, torch.float16: 4 * 2.0 ** -11, torch.float32: 1e-5}[dt]
+    tol = {torch.bfloat16: 2 * 2.0 ** -8, torch.float16: 4 * 2.0 ** -11, torch.float32: 1e-5}[dt]
     for chunk_bytes in (1 << 31, 512 * V * x.element_size()):  # one chunk, and chunks of 512 rows
         monkeypatch.setattr(CE, "_CHUNK_BYTES", chunk_bytes)
         got = CE.LigerFusedLinearCrossEntropyFunction.apply(x, w, t, b, None, -100, 0.0, 0.0, "mean", None, False, accum)[0]
@@ -118,4 +120,5 @@ def test_lm_loss_layouts(rows, V, bias, dt, accum, monkeypatch):
             assert a.shape == r.shape and a.is_contiguous()
             assert (a.float() - r).norm() <= tol * r.norm() + 1e-12, (chunk_bytes, a.shape)
         with torch.no_grad():  # no gradients wanted: the loss alone
-            assert float(CE.LigerFusedLinearCrossEntropyFunction.apply(x.detach(), w.detach(), t)[0]) > 0 or bias
+            alone = CE.LigerFusedLinearCrossEntropyFunction.apply(x.detach(), w.detach(), t, b.detach() if bias else None)[0]
+            assert abs(float(alone) - float(loss)) <= 2e-5 * abs(float(loss)) + (0 if dt == torch.float32 else 1e-3)
