@@ -332,17 +332,15 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 && D == 64) ? (BN == 32 ? (TR 
         bool act[NST];
         // a band chunk some row sees is computed whole under the window mask (a subtile wholly
         // outside every window scores -inf and adds zeros: cheaper than the branches that
-        // would skip it; the training variant, whose edge terms cost more, skips it);
-        // landmark subtiles past the largest visible count are skipped
+        // would skip it); landmark subtiles past the largest visible count are skipped
         const bool cact = band ? (base <= whi && base + BN - 1 >= wlo) : true;
 #pragma unroll
         for (int stt = 0; stt < NST; ++stt) {
             const int a = base + stt * 16;
             act[stt] = band ? cact : (a < wcmax);
             if (!act[stt]) {
-                // an inactive band chunk of the inference variant adds nothing (both subtiles
-                // share its activity, so its dS is never read); a skipped subtile beside an
-                // active one adds zeros
+                // an inactive band chunk adds nothing (its subtiles share its activity, so its dS is
+                // never read); a skipped landmark subtile beside an active one adds zeros
                 if (!band) dS[stt] = floatx4{0.f, 0.f, 0.f, 0.f};
                 continue;
             }
@@ -437,7 +435,7 @@ __global__ __launch_bounds__(256, (sizeof(T) == 2 && D == 64) ? (BN == 32 ? (TR 
             const int ir = __shfl(vi, rr);
             return ir >= 0 ? dq0 + ir * rstride : (T*)nullptr;
         });
-    } else if (valid) {  // (the training variant's registers leave no room for the staging)
+    } else if (valid) {  // the training variant stores its rows from the accumulators, in 8-byte pieces
         T* drow = dq0 + i * rstride;
 #pragma unroll
         for (int dt = 0; dt < D / 16; ++dt) {
@@ -529,8 +527,10 @@ struct QLoader {
 //     partial rows j0 < lo_i <= j0+63   (see keys >= lo_i: one-sided mask);
 // rows with lo_i > j0 + 63 are skipped.  List order is row order, so the sum
 // order is fixed and results are deterministic.
-// four waves per SIMD for 16-bit head_dim 64 (32-row stages keep it free of spills; three with
-// the head loop of grouped heads, which needs more registers), two otherwise.
+// four waves per SIMD for 16-bit head_dim 64 (32-row stages keep the operator free of spills; the
+// one-head training variant holds 8 bytes of scratch: 16 heads x 32768 177 us, at three waves and
+// 129 VGPRs 199), three with the head loop of grouped heads, which needs more registers, two
+// otherwise.
 // TR: training variant -- fully visible rows must also see every key of the block
 // past their edge_keys edge-bias keys; other rows add the soft edge bias.
 // GQA: the key/value head has several query heads (swept in order); without it the

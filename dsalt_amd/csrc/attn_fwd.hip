@@ -184,9 +184,13 @@ __device__ __forceinline__ void band_edge(const AttnParams& p, const RowGroup& R
     }
 }
 
+// (head, sequence) pairs from which each XCD walks its pairs one at a time (fwd_kernel)
+constexpr int kPairOrderMin = 256;
+
 // One 256-thread block (4 waves; NW = 8 below: 512 threads) owns 64*RG query rows of one (head, sequence),
 // (two 16-row groups with 32-key chunks, 16-bit head_dim 64: held at four waves per SIMD, 128
-// VGPRs; the K and V^T operands of a chunk serve both groups of a wave)
+// VGPRs, three spilled in the training variant; the K and V^T operands of a chunk serve both
+// groups of a wave)
 // taken in the row plan's order; wave w owns the 16-row groups RG*w .. RG*w+RG-1
 // (each lane one query row per group).  The K and V^T operands fetched from
 // LDS for a subtile serve all of a wave's groups.
@@ -204,9 +208,6 @@ __device__ __forceinline__ void band_edge(const AttnParams& p, const RowGroup& R
 // serves twice the rows (head_dim 128, where the chunks' staging is most of the time).
 // (the 16-bit head_dim-128 training forward is held to four waves per SIMD: 128 VGPRs, no
 // spills, from 132 at three)
-// (head, sequence) pairs from which each XCD walks its pairs one at a time (fwd_kernel)
-constexpr int kPairOrderMin = 256;
-
 //
 // IP: each block makes its tile's row plan itself (plan_regs, by every wave; head 0's blocks also
 // write it to the plan buffer) instead of reading the one a launch before it wrote.
@@ -734,8 +735,8 @@ __global__ __launch_bounds__(64 * NW, ((sizeof(T) == 2 && D == 64 && RG == 2 && 
 //     windows up to 64 0.97-1.03x; 24576 tiles 0.94-1.03x, 16384 0.95-1.08x.  Grouped heads find
 //     their chunks in L2 (0.93-1.11x, 1.02x on average), and shorter sequences fill fewer of the
 //     128 rows (8192 tokens up to 1.04x, 512 1.12x, 64 1.23x).
-// The training variant keeps 64-row blocks: its two row groups are held to too few registers
-// (1.13-1.26x from 1536 tiles on).
+// The training variant keeps 64-row blocks: with two row groups and 64-key chunks it holds 170
+// VGPRs, two waves per SIMD (1536 to 16384 tiles 1.13-1.26x).
 // Sets of more than kSetSlots landmarks, and block-causal sets of a block_size that is not a
 // multiple of 64, take the default tiling's wide instantiation (variant bits ignored).
 constexpr int64_t kRg2Tiles = 6144, kRg2Len = 1024, kW8Tiles = 32768, kW8Len = 65536;

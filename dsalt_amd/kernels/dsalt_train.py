@@ -66,9 +66,9 @@ class DSALTTrainFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, grad_out):
         q, k, v, out, lse, idx_s, logw_s, perm, w_c, cu_i, plan = ctx.saved_tensors
+        go = grad_out if ctx.head_dim == q.shape[-1] else pad_head_dim(grad_out.to(q.dtype), q.shape[-1])
         dq, dk, dv, dlogw, d_w = ops.train_backward(
-            grad_out if ctx.head_dim == q.shape[-1] else pad_head_dim(grad_out.to(q.dtype), q.shape[-1]), q, k, v, out, lse, w_c, cu_i, idx_s, logw_s,
-            tau_win=ctx.tau_win,
+            go, q, k, v, out, lse, w_c, cu_i, idx_s, logw_s, tau_win=ctx.tau_win,
             win_edge=ctx.win_edge, scale=ctx.scale, max_seqlen=ctx.max_seqlen,
             want_dlogw=ctx.needs_input_grad[4], plan=plan, variant=ctx.variant)
         d_logw = None
