@@ -1232,7 +1232,8 @@ __device__ __forceinline__ int find_slot(const int32_t* set, int K, int pos) {
 // heads' sets and then partials in flight at a time, and four waves share a row of at least
 // kSumSplit chunks while the rows with sums to add (about rows / heads of a group) are fewer than
 // kSumFill, two waves per SIMD; from there on one wave a row keeps the memory busy (2048 owners of
-// 32 chunks: 9.9 us with one wave a row, 13.0 with four; 512 owners of 16 chunks: 11.5 and 7.0).  16/4 heads x 8192, head_dim 128: 26.6 -> 13.8 us; 8/2 heads, 5 short sequences: 13.9 -> 7.2.
+// 32 chunks: 9.9 us with one wave a row, 13.0 with four; 512 owners of 16 chunks: 11.5 and 7.0).
+// 16/4 heads x 8192, head_dim 128: 26.6 -> 13.8 us; 8/2 heads, 5 short sequences: 13.9 -> 7.2.
 constexpr int kSumSplit = 8, kSumFill = 2048;
 
 template <typename T, int D, int WPR>
@@ -1287,12 +1288,16 @@ __global__ __launch_bounds__(256) void bwd_lmk_sum_kernel(AttnParams p) {
     const int c0 = part * cq, c1 = min(p.n_chunks, c0 + cq);
     const float* pk = p.part_k + lane * CPL;
     const float* pv = p.part_v + lane * CPL;
-    // partials of N slots (rows of the partials, -1: none), U chunks of each in flight
+    // partials of N slots (rows of the partials, -1: none), U chunks of each in flight; a single
+    // slot's chunks are added to the running sums one by one
     auto add_slots = [&](auto n_tag, auto u_tag, const int64_t* rows) {
         constexpr int N = decltype(n_tag)::value, U = decltype(u_tag)::value;
         vec hk[N], hv[N];
 #pragma unroll
-        for (int n = 0; n < N; ++n) hk[n] = hv[n] = (vec)(0.f);
+        for (int n = 0; n < N; ++n) {
+            hk[n] = N == 1 ? sk : (vec)(0.f);
+            hv[n] = N == 1 ? sv : (vec)(0.f);
+        }
         for (int ch0 = c0; ch0 < c1; ch0 += U) {
             vec ak[N][U], av[N][U];
 #pragma unroll
@@ -1317,8 +1322,8 @@ __global__ __launch_bounds__(256) void bwd_lmk_sum_kernel(AttnParams p) {
         }
 #pragma unroll
         for (int n = 0; n < N; ++n) {
-            sk += hk[n];
-            sv += hv[n];
+            sk = N == 1 ? hk[n] : sk + hk[n];
+            sv = N == 1 ? hv[n] : sv + hv[n];
         }
     };
     typedef std::integral_constant<int, 1> one;
