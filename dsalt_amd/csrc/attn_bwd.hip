@@ -1234,7 +1234,12 @@ __device__ __forceinline__ int find_slot(const int32_t* set, int K, int pos) {
 // kSumFill, two waves per SIMD; from there on one wave a row keeps the memory busy (2048 owners of
 // 32 chunks: 9.9 us with one wave a row, 13.0 with four; 512 owners of 16 chunks: 11.5 and 7.0).
 // 16/4 heads x 8192, head_dim 128: 26.6 -> 13.8 us; 8/2 heads, 5 short sequences: 13.9 -> 7.2.
+// From kSumMany rows on the waves' instructions count, not one row's latency: empty slots leave on
+// the position alone, and a head on its own keys reads its neighbouring slots instead of searching
+// (16 heads of 128 slots: 512 sequences of 512 tokens 1037 -> 523 us, 128 of 2048 257 -> 152; 4096 rows
+// of short sequences 9.3 -> 8.1, 2048 rows of 32 chunks 12 -> 13.6).
 constexpr int kSumSplit = 8, kSumFill = 2048;
+constexpr uint32_t kSumMany = 1 << 12;
 
 template <typename T, int D, int WPR>
 __global__ __launch_bounds__(256) void bwd_lmk_sum_kernel(AttnParams p) {
@@ -1242,17 +1247,36 @@ __global__ __launch_bounds__(256) void bwd_lmk_sum_kernel(AttnParams p) {
     typedef float vec __attribute__((ext_vector_type(CPL)));
     __shared__ __attribute__((aligned(16))) vec red[WPR > 1 ? 2 * 4 * 64 : 1];
     const int K = p.k_lmk, lane = threadIdx.x & 63, wave = uniform((int)threadIdx.x >> 6);
-    const int64_t row = WPR > 1 ? (int64_t)blockIdx.x : (int64_t)blockIdx.x * 4 + wave;  // (h, s, slot)
+    const uint32_t rows_all = (uint32_t)p.n_heads * p.num_seqs * K;
+    const uint32_t row = WPR > 1 ? blockIdx.x : blockIdx.x * 4 + wave;  // (h, s, slot)
     const int part = WPR > 1 ? wave : 0;
-    if (row >= (int64_t)p.n_heads * p.num_seqs * K) return;
-    const int sl = (int)(row % K);
-    const int s = (int)((row / K) % p.num_seqs);
-    const int h = (int)(row / ((int64_t)K * p.num_seqs));
+    if (row >= rows_all) return;
+    const int64_t cstride = rows_all;
+    auto write_bias = [&]() {
+        if (!p.d_bias || part > 0) return;
+        float sb = 0.f;
+        for (int ch0 = 0; ch0 < p.n_chunks; ch0 += 64) {  // a chunk per lane, added in chunk order
+            const int n = min(64, p.n_chunks - ch0);
+            const float v = lane < n ? p.part_b[(ch0 + lane) * cstride + row] : 0.f;
+            for (int u = 0; u < n; ++u) sb += __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), u));
+        }
+        if (lane == 0) p.d_bias[row] = sb;
+    };
+    const int pos = p.lmk[row];  // (one set per head and sequence)
+    const bool many = rows_all >= kSumMany;
+    if (many) {
+        write_bias();
+        if (uniform(pos) < 0) return;
+    }
+    const int sl = (int)(row % (uint32_t)K);
+    const uint32_t set_no = row / (uint32_t)K;
+    const int s = (int)(set_no % (uint32_t)p.num_seqs);
+    const int h = (int)(set_no / (uint32_t)p.num_seqs);
     const int rep = p.n_heads / p.n_kv_heads, kvh = h / rep, hend = (kvh + 1) * rep;
     auto set_of = [&](int hh) { return p.lmk + (((int64_t)hh * p.num_seqs + s) * p.n_sets) * K; };
     // the first batch of sets and the band sums are requested with the position: one latency
     constexpr int HB = 4;
-    const bool wide = K > 128;
+    const bool wide = K > 128 || (many && rep == 1);
     int v0[HB], v1[HB];
     auto load_sets = [&](int hb) {
 #pragma unroll
@@ -1263,22 +1287,12 @@ __global__ __launch_bounds__(256) void bwd_lmk_sum_kernel(AttnParams p) {
         }
     };
     if (!wide) load_sets(kvh * rep);
-    const int pos = set_of(h)[sl];
-    const int64_t half = (int64_t)p.n_heads * p.num_seqs * K * D;
-    const int64_t so = row * D + lane * CPL;
+    const int64_t half = (int64_t)rows_all * D;
+    const int64_t so = (int64_t)row * D + lane * CPL;
     vec sk = *(const vec*)(p.lmk_stage + so), sv = *(const vec*)(p.lmk_stage + half + so);
     int st, len;
     seq_bounds(p.cu, s, p.total_len, p.max_seqlen, st, len);
-    const int64_t cstride = (int64_t)p.n_heads * p.num_seqs * K;
-    if (p.d_bias && part == 0) {
-        float sb = 0.f;
-        for (int ch0 = 0; ch0 < p.n_chunks; ch0 += 64) {  // a chunk per lane, added in chunk order
-            const int n = min(64, p.n_chunks - ch0);
-            const float v = lane < n ? p.part_b[(ch0 + lane) * cstride + row] : 0.f;
-            for (int u = 0; u < n; ++u) sb += __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), u));
-        }
-        if (lane == 0) p.d_bias[row] = sb;
-    }
+    if (!many) write_bias();
     if (pos < 0 || pos >= len) return;
     if (part > 0) {  // the band sums enter once
         sk = (vec)(0.f);
@@ -1334,7 +1348,8 @@ __global__ __launch_bounds__(256) void bwd_lmk_sum_kernel(AttnParams p) {
     auto add_copies = [&](int hh, int slot0, int n) {
         for (int slot = slot0; slot < slot0 + n; ++slot) {
             const int64_t r = prow(hh, slot);
-            add_slots(one{}, std::integral_constant<int, 8>{}, &r);
+            if (c1 - c0 > 2) add_slots(one{}, std::integral_constant<int, 8>{}, &r);
+            else add_slots(one{}, std::integral_constant<int, 2>{}, &r);
         }
     };
     // only the owner of the row goes on: no earlier head of the group holds the position, and
