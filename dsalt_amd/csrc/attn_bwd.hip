@@ -1475,14 +1475,17 @@ static hipError_t bwd_run(const AttnParams& p, bool plan_given, hipStream_t stre
         if (p.w_cont) DSALT_LAUNCH("bwd_dq", (bwd_dq_kernel<T, D, BN, true>), dim3(total), dim3(256), 0, stream, p);
         else DSALT_LAUNCH("bwd_dq", (bwd_dq_kernel<T, D, BN, false>), dim3(total), dim3(256), 0, stream, p);
     }
-    // grouped heads, 16-bit head_dim 64, two or four to a key/value head: side by side (the whole
-    // backward, 4/1 heads x 1024: 54.6 -> 34.7 us, 16/4 heads x 8192: 147.4 -> 132.0, 16/4 x 32768:
-    // 399.7 -> 393.0, 16/8 x 32768: 397.9 -> 382.9).  Four heads of the training variant, whose edge
-    // terms keep every wave busier, gain until the blocks fill the chip several times over (1024
-    // blocks 318.5 -> 299.4 us, 2048 blocks 519.4 -> 531.7): from 2048 blocks on they stay in order.
+    // grouped heads, 16-bit head_dim 64, two or four to a key/value head: side by side.  A CU holds
+    // two blocks of two heads, one of four, and three of the head loop, whose round takes about twice
+    // as long.  Two heads gain at every size (dK/dV alone: 128 blocks 0.62-0.78x the loop's time, 4096
+    // 0.87-0.96x, 16384 0.92-0.96x; 16/8 heads x 32768 161.6 -> 142.2 us).  Four heads take the rounds
+    // of 256 blocks they fill against twice those of 768 (windows up to 64 .. 512, operator and training
+    // variant alike): up to 256 blocks 0.48-0.65x, 512 0.80-0.95x, 564 to 768 1.01-1.20x, 846 to 1024
+    // 0.82-1.02x, 2048 1.01-1.19x, 8192 1.10-1.30x (16/4 heads x 8192 55.8 -> 46.2 us).
     const int rep = p.n_heads / p.n_kv_heads;
     constexpr bool kSide = sizeof(T) == 2 && D == 64;
-    if (kSide && (rep == 2 || (rep == 4 && !(p.w_cont && total_kv >= 2048)))) {
+    const bool fills = ceil_div(total_kv, 256) <= 2 * ceil_div(total_kv, 768);
+    if (kSide && (rep == 2 || (rep == 4 && fills))) {
         if constexpr (kSide) {
             if (rep == 2) {
                 if (p.w_cont) DSALT_LAUNCH("bwd_dkdv", (bwd_dkdv_kernel<T, D, true, false, 2>), dim3(total_kv), dim3(512), 0, stream, p);

@@ -115,7 +115,9 @@ def test_plan_made_by_the_blocks(lens, H, D, dt):
     ([3000], 128, 32, 64, 70, torch.bfloat16),            # few chunks: one wave a row
     ([7200], 32, 16, 64, 128, torch.bfloat16),            # eight chunks, 2048 owner rows: one wave a row
     ([7200], 32, 16, 64, 127, torch.bfloat16),            # 2032 owner rows: four waves a row
-    ([4097], 128, 32, 64, 20, torch.bfloat16),            # 2080 blocks: the training heads of a group in order
+    ([4097], 128, 32, 64, 20, torch.bfloat16),            # 2080 blocks: the four heads of a group in order
+    ([4161], 32, 8, 64, 20, torch.bfloat16),              # 528 blocks, likewise
+    ([6145], 32, 8, 64, 20, torch.float16),               # 776 blocks: side by side in their fourth round
     ([70] * 60 + [0, 1, 64, 65], 8, 4, 64, 20, torch.bfloat16),  # many rows of short sequences
     ([520, 333], 4, 1, 64, 9, torch.float32),
 ])
