@@ -717,9 +717,8 @@ __global__ __launch_bounds__(64 * NW, ((sizeof(T) == 2 && D == 64 && RG == 2 && 
 // row groups per wave (FWD_RG2, same condition) or 64-key chunks instead of 32 (FWD_BN64;
 // ignored with FWD_RG2).  The bit of the chunk length a head_dim has anyway (FWD_BN64 at 64,
 // FWD_BN32 at 128) asks for its 64-row blocks at any size; fp32 takes its single compiled
-// tiling.  With no forward bit set the call picks by its work
-// in 64-row tiles, tokens x heads / 64, among tilings whose outputs are the same bit for bit: equal
-// key chunks on the same boundaries, so the same running maxima and roundings of P (32-key chunks at
+// tiling.  With no forward bit set the call picks by its work in 64-row tiles, tokens x heads / 64,
+// among tilings whose outputs are the same bit for bit: equal key chunks on the same boundaries, so the same running maxima and roundings of P (32-key chunks at
 // head_dim 64 round P against other maxima, 2.18e-3 against 2.13e-3 from the float64 result at
 // 16 heads x 32768, and are left to the caller's bit).  Against the 64-row tiling, row plan given,
 // windows up to 64 .. 512, 16 .. 256 landmarks:
@@ -732,9 +731,8 @@ __global__ __launch_bounds__(64 * NW, ((sizeof(T) == 2 && D == 64 && RG == 2 && 
 //   head_dim 128: FWD_8W from kW8Tiles on where every head has its own keys and sequences hold kW8Len
 //     tokens on average, so that staging the key chunks bounds the kernel: 32768 tiles, windows up
 //     to 256 or 512 0.92-0.99x (16 heads x 131072, windows up to 512, 256 landmarks: 1225 -> 1159 us),
-//     windows up to 64 0.97-1.03x; 24576 tiles 0.94-1.03x, 16384 0.95-1.08x.  Grouped heads find
-//     their chunks in L2 (0.93-1.11x, 1.02x on average), and shorter sequences fill fewer of the
-//     128 rows (8192 tokens up to 1.04x, 512 1.12x, 64 1.23x).
+//     windows up to 64 0.97-1.03x; 24576 tiles 0.94-1.03x, 16384 0.95-1.08x.  Grouped heads
+//     0.93-1.11x, 1.02x on average; shorter sequences 8192 tokens up to 1.04x, 512 1.12x, 64 1.23x.
 // The training variant keeps 64-row blocks: with two row groups and 64-key chunks it holds 170
 // VGPRs, two waves per SIMD (1536 to 16384 tiles 1.13-1.26x).
 // Sets of more than kSetSlots landmarks, and block-causal sets of a block_size that is not a
@@ -768,11 +766,13 @@ FwdTile fwd_tile(const AttnParams& p, bool train) {
     return t;
 }
 
-// Calls of up to kInlineTiles 64-row tiles (x heads) make the plan in the attention's own blocks: the
-// launch before costs its own latency, a plan per block and head under a microsecond of each
-// round of blocks.  Plan and forward, us (graph replay, so without the launch's 3 us on the host):
-// 32 tiles 12.1 -> 10.1, 512 14.7 -> 13.3, 1024 19.7 -> 19.1, 1375 39.2 -> 39.7; head_dim 128: 256
-// tiles 14.5 -> 12.4, 1024 24.7 -> 22.9, 8192 125 -> 136; float32: 512 29.1 -> 26.8, 2048 72.8 -> 74.5.
+// Calls of up to kInlineTiles blocks (64-row tiles of every sequence x heads, those past a shorter
+// sequence's end included) make the plan in the attention's own blocks: the launch before costs its
+// own latency, a plan per block and head under a microsecond of each round of blocks.  Plan and
+// forward, us (graph replay, so without the launch's 3 us on the host): 32 blocks 12.1 -> 10.1, 512
+// 14.7 -> 13.3, 1024 19.7 -> 19.1, 1375 39.2 -> 39.7; head_dim 128: 256 14.5 -> 12.4, 1024 24.7 -> 22.9,
+// 8192 125 -> 136; float32: 512 29.1 -> 26.8, 2048 72.8 -> 74.5.  Blocks without rows count as well: one
+// sequence of 2000 tokens beside 1000 of 5, 4 heads, 118 -> 334 us.
 constexpr int64_t kInlineTiles = 1024;
 
 template <typename T, int D, bool TR>
@@ -781,7 +781,7 @@ static hipError_t fwd_run(const AttnParams& p, bool plan_ready, hipStream_t stre
     const FwdTile t = fwd_tile(p, TR);
     const dim3 grid(p.n_heads * p.num_seqs * ceil_div(p.n_tiles, t.rows / 64)), block(64 * t.waves);
     if (!plan_ready) {
-        const int64_t tiles = (int64_t)p.total_len * p.n_heads / 64;
+        const int64_t tiles = (int64_t)p.n_heads * p.num_seqs * p.n_tiles;
         if (t.rows == 64 && t.keys == BN && !t.multi && tiles <= kInlineTiles) {
             DSALT_LAUNCH("attn_fwd", (fwd_kernel<T, D, BN, 1, TR, false, 4, true>), grid, block, 0, stream, p);
             return hipGetLastError();
