@@ -1475,17 +1475,25 @@ static hipError_t bwd_run(const AttnParams& p, bool plan_given, hipStream_t stre
         if (p.w_cont) DSALT_LAUNCH("bwd_dq", (bwd_dq_kernel<T, D, BN, true>), dim3(total), dim3(256), 0, stream, p);
         else DSALT_LAUNCH("bwd_dq", (bwd_dq_kernel<T, D, BN, false>), dim3(total), dim3(256), 0, stream, p);
     }
-    // grouped heads, 16-bit head_dim 64, two or four to a key/value head: side by side.  A CU holds
-    // two blocks of two heads, one of four, and three of the head loop, whose round takes about twice
-    // as long.  Two heads gain at every size (dK/dV alone: 128 blocks 0.62-0.78x the loop's time, 4096
-    // 0.87-0.96x, 16384 0.92-0.96x; 16/8 heads x 32768 161.6 -> 142.2 us).  Four heads take the rounds
-    // of 256 blocks they fill against twice those of 768 (windows up to 64 .. 512, operator and training
-    // variant alike): up to 256 blocks 0.48-0.65x, 512 0.80-0.95x, 564 to 768 1.01-1.20x, 846 to 1024
-    // 0.82-1.02x, 2048 1.01-1.19x, 8192 1.10-1.30x (16/4 heads x 8192 55.8 -> 46.2 us).
+    // grouped heads, 16-bit head_dim 64, two or four to a key/value head: side by side where their
+    // rounds of blocks pay.  A CU holds two blocks of two heads, one of four, and three of the head
+    // loop, so a round is 512, 256 and 768 blocks; the loop's takes 1.4 and 1.8 times as long.  dK/dV
+    // against the loop's time, operator and training variant, windows up to 64 .. 512:
+    //   two heads: up to 512 blocks 0.62-0.90x, 513 to 768 0.87-1.10x, from there on 0.78-0.97x
+    //     (16/8 heads x 32768 161.6 -> 142.2 us);
+    //   four: up to 256 blocks 0.48-0.65x, 512 0.78-0.95x, 564 to 768 1.01-1.20x, 846 to 1024 0.82-1.02x,
+    //     2048 1.01-1.19x, 8192 1.10-1.30x (16/4 heads x 8192 55.8 -> 46.2 us).
+    // Past one round, blocks without rows or of short sequences cost the larger blocks more than
+    // the loop's (half of the tiles empty 0.92-1.12x, nearly all 1.4-2.3x; sequences of 64 tokens
+    // 1.05-1.6x, of 128 0.90-0.98x).
     const int rep = p.n_heads / p.n_kv_heads;
     constexpr bool kSide = sizeof(T) == 2 && D == 64;
-    const bool fills = ceil_div(total_kv, 256) <= 2 * ceil_div(total_kv, 768);
-    if (kSide && (rep == 2 || (rep == 4 && fills))) {
+    // blocks with rows: at least `least`, at most `most`
+    const int64_t least = (int64_t)p.n_kv_heads * ceil_div(p.total_len, 64), most = least + (int64_t)p.n_kv_heads * p.num_seqs;
+    const bool dense = 2 * least >= total_kv, lng = p.total_len >= (int64_t)128 * p.num_seqs;
+    const bool side2 = total_kv <= 512 || (dense && lng && (most <= 512 || least > 768));
+    const bool side4 = total_kv <= 256 || (lng && (total_kv <= 512 || (dense && most <= 512) || (least > 768 && total_kv <= 1024)));
+    if (kSide && ((rep == 2 && side2) || (rep == 4 && side4))) {
         if constexpr (kSide) {
             if (rep == 2) {
                 if (p.w_cont) DSALT_LAUNCH("bwd_dkdv", (bwd_dkdv_kernel<T, D, true, false, 2>), dim3(total_kv), dim3(512), 0, stream, p);
