@@ -1235,10 +1235,12 @@ __device__ __forceinline__ int find_slot(const int32_t* set, int K, int pos) {
 // 32 chunks: 9.9 us with one wave a row, 13.0 with four; 512 owners of 16 chunks: 11.5 and 7.0).
 // 16/4 heads x 8192, head_dim 128: 26.6 -> 13.8 us; 8/2 heads, 5 short sequences: 13.9 -> 7.2.
 // From kSumMany rows on the waves' instructions count, not one row's latency: empty slots leave on
-// the position alone, and a head on its own keys reads its neighbouring slots instead of searching
-// (16 heads of 128 slots: 512 sequences of 512 tokens 1037 -> 523 us, 128 of 2048 257 -> 152; 4096 rows
-// of short sequences 9.3 -> 8.1, 2048 rows of 32 chunks 12 -> 13.6).
-constexpr int kSumSplit = 8, kSumFill = 2048;
+// the position alone, and a head on its own keys looks at its neighbouring slots instead of searching
+// (16 heads of 128 slots: 512 sequences of 512 tokens 1037 -> 493 us, 128 of 2048 254 -> 127, 8 of 8192
+// 23.3 -> 21.0; 4096 rows of short sequences 9.3 -> 8.1, 2048 rows of 32 chunks 12 -> 13.6), but with
+// more than kSumManyChunks chunks, whose scattered partials lose by more waves at once (308K rows, a
+// sixth of them filled, 59 chunks: 778 us searching, 1015 without).
+constexpr int kSumSplit = 8, kSumFill = 2048, kSumManyChunks = 16;
 constexpr uint32_t kSumMany = 1 << 12;
 
 template <typename T, int D, int WPR>
@@ -1262,7 +1264,8 @@ __global__ __launch_bounds__(256) void bwd_lmk_sum_kernel(AttnParams p) {
         }
         if (lane == 0) p.d_bias[row] = sb;
     };
-    const int pos = p.lmk[row];  // (one set per head and sequence)
+    // the slot's position and its neighbours' (one set per head and sequence)
+    const int pos = p.lmk[row], before = p.lmk[max(row, 1u) - 1], after = p.lmk[min(row + 1, rows_all - 1)];
     const bool many = rows_all >= kSumMany;
     if (many) {
         write_bias();
@@ -1276,7 +1279,7 @@ __global__ __launch_bounds__(256) void bwd_lmk_sum_kernel(AttnParams p) {
     auto set_of = [&](int hh) { return p.lmk + (((int64_t)hh * p.num_seqs + s) * p.n_sets) * K; };
     // the first batch of sets and the band sums are requested with the position: one latency
     constexpr int HB = 4;
-    const bool wide = K > 128 || (many && rep == 1);
+    const bool wide = K > 128 || (many && rep == 1 && p.n_chunks <= kSumManyChunks);
     int v0[HB], v1[HB];
     auto load_sets = [&](int hb) {
 #pragma unroll
@@ -1377,15 +1380,15 @@ __global__ __launch_bounds__(256) void bwd_lmk_sum_kernel(AttnParams p) {
             }
         }
     } else {
-        const int32_t* set = set_of(h);
-        if (sl > 0 && set[sl - 1] == pos) return;
+        if (sl > 0 && before == pos) return;
         for (int hh = kvh * rep; hh < h; ++hh)
             if (find_slot(set_of(hh), K, pos) >= 0) return;
         for (int hh = h; hh < hend; ++hh) {
             const int32_t* hset = set_of(hh);
             const int first = hh == h ? sl : find_slot(hset, K, pos);
-            int n = 0;
-            while (first >= 0 && first + n < K && hset[first + n] == pos) ++n;
+            int n = hh == h ? 1 : 0;
+            if (hh != h || (sl + 1 < K && after == pos))
+                while (first >= 0 && first + n < K && hset[first + n] == pos) ++n;
             add_copies(hh, first, n);
         }
     }

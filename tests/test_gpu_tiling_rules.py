@@ -89,7 +89,8 @@ def test_forward_tiling_by_size(lens, H, G, D, dt, block):
     assert (lse[:, heads] - rlse).abs().max() <= UNIT[dt] + 1e-5
 
 
-@pytest.mark.parametrize("lens,H", [([8190], 8), ([8200], 8), ([700, 0, 1, 64, 65], 4), ([700, 0, 1, 64, 65], 160)])
+@pytest.mark.parametrize("lens,H", [([8190], 8), ([8200], 8), ([700, 0, 1, 64, 65], 4), ([700, 0, 1, 64, 65], 160),
+                                    ([2000] + [5] * 100, 4)])
 @pytest.mark.parametrize("D,dt", [(64, torch.bfloat16), (128, torch.float16), (64, torch.float32)])
 def test_plan_made_by_the_blocks(lens, H, D, dt):
     """The row plan of the attention's own blocks (small calls) is the selection's, byte for byte,
@@ -119,6 +120,8 @@ def test_plan_made_by_the_blocks(lens, H, D, dt):
     ([4161], 32, 8, 64, 20, torch.bfloat16),              # 528 blocks, likewise
     ([6145], 32, 8, 64, 20, torch.float16),               # 776 blocks: side by side in their fourth round
     ([70] * 60 + [0, 1, 64, 65], 8, 4, 64, 20, torch.bfloat16),  # many rows of short sequences
+    ([30] * 300, 8, 4, 64, 4, torch.bfloat16),            # 1200 blocks of one short sequence: heads in order
+    ([9300] + [0, 40] * 60, 8, 8, 64, 6, torch.bfloat16),  # many rows, most of them empty, 10 chunks
     ([520, 333], 4, 1, 64, 9, torch.float32),
 ])
 @pytest.mark.parametrize("train", [False, True])
